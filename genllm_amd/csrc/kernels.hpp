@@ -122,7 +122,17 @@ constexpr int kDecodeMergeKernel = 0, kDecodeMergeFused = 1;
 int set_decode_tuning(int pages_per_split, int merge, int heads_per_wg);
 int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws);
 int launch_paged_decode(const AttnParams& p, int head_dim, hipStream_t stream);
-int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream);
+// Batch entries of one prefill launch: element strides between entries (the
+// kv stride is 0 where every entry attends the same cache).
+struct PrefillBatch {
+    int32_t n = 1;
+    int64_t q_stride = 0, o_stride = 0, kv_stride = 0;
+};
+// ws (may be null: no launch is split): scratch for the partials of a
+// key-split launch, prefill_workspace_bytes for the most keys a call may have.
+size_t prefill_workspace_bytes(int head_dim, int64_t max_tokens);
+int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream, const PrefillBatch& b = {},
+                         float* ws = nullptr, size_t ws_bytes = 0);
 
 int launch_rms_norm(uint16_t* out, const uint16_t* x, const float* w, int64_t rows, int hidden, float eps,
                     hipStream_t stream);

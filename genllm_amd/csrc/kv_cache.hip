@@ -114,6 +114,11 @@ struct LayerState {
     int32_t* h_ids = nullptr;
     int32_t max_blocks = 0;
     size_t block_bytes = 0;
+    // Partials of key-split prefill chunks (prefill_workspace_bytes), or null:
+    // such a chunk then runs unsplit.  Its own for each layer, so that chunks of
+    // different layers may run on different streams.
+    float* prefill_ws = nullptr;
+    size_t prefill_ws_bytes = 0;
     // Device-position decode (graph-capturable steps): the control block
     // {pos, limit, arrivals, error} follows the device page table.  Between
     // genllm_kv_stage_decode and genllm_kv_sync_decode the device owns the
@@ -143,7 +148,7 @@ struct genllm_kv {
     void* ws = nullptr;
     size_t ws_bytes = 0;
     std::vector<void*> pinned;     // every h_ids buffer, freed at destroy
-    std::vector<void*> tables;     // every device page table, freed at destroy
+    std::vector<void*> tables;     // every device page table and prefill scratch, freed at destroy
     bool uploads_pending = false;  // async table uploads from h_ids may be in flight
 };
 
@@ -353,9 +358,10 @@ int prepare_attention(AttnParams& p, int head_dim, genllm_kv* kv) {
     return GENLLM_OK;
 }
 
-int launch_attention(const AttnParams& p, int head_dim, hipStream_t stream) {
+int launch_attention(const AttnParams& p, const LayerState& s, int head_dim, hipStream_t stream,
+                     const PrefillBatch& batch = {}) {
     if (p.G * p.S <= 16) return launch_paged_decode(p, head_dim, stream);
-    return launch_paged_prefill(p, head_dim, stream);
+    return launch_paged_prefill(p, head_dim, stream, batch, s.prefill_ws, s.prefill_ws_bytes);
 }
 
 }  // namespace
@@ -464,6 +470,18 @@ extern "C" int genllm_kv_reserve_layer(genllm_kv* kv, int32_t layer, int32_t max
         (void)hipHostFree(staging);
         kv->cursor = cursor0;
         return rc;
+    }
+    const size_t pw_need = elem_size(s.dtype) == 2 ? prefill_workspace_bytes(s.head_dim, int64_t(max_blocks) * kPage) : 0;
+    if (pw_need > s.prefill_ws_bytes) {
+        // without it (no memory left) the layer's chunks run unsplit
+        void* pw = nullptr;
+        if (hipMalloc(&pw, pw_need) == hipSuccess) {
+            s.prefill_ws = static_cast<float*>(pw);
+            s.prefill_ws_bytes = pw_need;
+            kv->tables.push_back(pw);
+        } else {
+            (void)hipGetLastError();
+        }
     }
     kv->tables.push_back(table);
     kv->pinned.push_back(staging);
@@ -725,7 +743,9 @@ extern "C" int genllm_paged_attention(genllm_kv* kv, int32_t layer, const void* 
             p.upd.v[i] = ap.upd.v[i];
         }
     }
-    if (int rc = launch_attention(p, head_dim, st)) {
+    // Longer chunks take every batch entry in one launch.
+    const int64_t entry = int64_t(n_q_heads) * seq_len * head_dim;
+    if (int rc = launch_attention(p, *s, head_dim, st, PrefillBatch{batch, entry, entry, 0})) {
         if (fuse) undo_append(*s, undo);  // nothing ran: the fused append is part of this launch
         return rc;
     }
@@ -734,16 +754,15 @@ extern "C" int genllm_paged_attention(genllm_kv* kv, int32_t layer, const void* 
     // above took the first entry's K/V rows, as append_kv_from_tensor reads
     // K->data for n_kv_heads x seq_len rows): attention only, after the first
     // entry's launch has written the new rows and page ids.
-    if (batch > 1) {
+    if (fuse && batch > 1) {
         AttnParams pb = p;
         pb.k_new = pb.v_new = nullptr;
         pb.new_from = INT32_MAX;
         pb.upd.count = 0;
-        const int64_t entry = int64_t(n_q_heads) * seq_len * head_dim;
         for (int32_t b = 1; b < batch; ++b) {
             pb.q = p.q + b * entry;
             pb.out = p.out + b * entry;
-            if (int rc = launch_attention(pb, head_dim, st)) return rc;
+            if (int rc = launch_attention(pb, *s, head_dim, st)) return rc;
         }
     }
     return GENLLM_OK;
@@ -857,7 +876,7 @@ extern "C" int genllm_paged_attention_step(genllm_kv* kv, int32_t layer, const v
     p.step = s->d_step;
     if (int rc = prepare_attention(p, head_dim, kv)) return rc;
     fuse_append(p, *s, k, v, seq_len, head_dim, 0);
-    return launch_attention(p, head_dim, as_stream(stream));
+    return launch_attention(p, *s, head_dim, as_stream(stream));
 }
 
 
@@ -1215,7 +1234,7 @@ extern "C" int genllm_paged_decode_noalloc(const void* q, int64_t q_head_stride,
 // Non-paged attention (FlashAttentionImpl, attention.cpp:39-121): the prefill
 // kernel reading K/V straight from the [B][Hkv][S][D] tensors -- page i of a
 // head is rows 16i..16i+15 of that head, so no block table is involved.  Query
-// s attends keys 0..s (causal) or all S keys; one launch per batch entry.
+// s attends keys 0..s (causal) or all S keys; one launch for all batch entries.
 extern "C" int genllm_flash_attention(const void* q, const void* k, const void* v, void* out, int32_t batch,
                                       int32_t n_q_heads, int32_t seq_len, int32_t n_kv_heads, int32_t head_dim,
                                       int32_t n_kv_groups, float scale, int32_t causal, void* stream) {
@@ -1228,30 +1247,29 @@ extern "C" int genllm_flash_attention(const void* q, const void* k, const void* 
         return fail(GENLLM_ERR_INVALID, "flash_attention: scale must be finite and >= 0");
     if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 8))
         return fail(GENLLM_ERR_INVALID, "flash_attention: tensors must be 16-byte aligned");
+    if (batch == 0 || seq_len == 0) return GENLLM_OK;
     const int64_t D = head_dim, S = seq_len;
-    for (int32_t b = 0; b < batch && seq_len > 0; ++b) {
-        AttnParams p;
-        p.q = static_cast<const uint16_t*>(q) + int64_t(b) * n_q_heads * S * D;
-        p.q_head_stride = S * D;
-        p.q_tok_stride = D;
-        p.out = static_cast<uint16_t*>(out) + int64_t(b) * n_q_heads * S * D;
-        p.o_head_stride = S * D;
-        p.o_tok_stride = D;
-        p.k_pool = static_cast<const uint16_t*>(k) + int64_t(b) * n_kv_heads * S * D;
-        p.v_pool = static_cast<const uint16_t*>(v) + int64_t(b) * n_kv_heads * S * D;
-        p.k_ids = p.v_ids = nullptr;
-        p.n_pages = int32_t((S + kPage - 1) / kPage);
-        p.n_cached = seq_len;
-        p.S = seq_len;
-        p.Hq = n_q_heads;
-        p.Hkv = n_kv_heads;
-        p.G = n_kv_groups;
-        p.scale_log2 = scale * kLog2e;
-        p.causal = causal != 0;
-        p.page_elems = kPage * D;
-        p.kv_row = D;
-        p.kv_head_stride = S * D;
-        if (int rc = launch_paged_prefill(p, head_dim, as_stream(stream))) return rc;
-    }
-    return GENLLM_OK;
+    AttnParams p;
+    p.q = static_cast<const uint16_t*>(q);
+    p.q_head_stride = S * D;
+    p.q_tok_stride = D;
+    p.out = static_cast<uint16_t*>(out);
+    p.o_head_stride = S * D;
+    p.o_tok_stride = D;
+    p.k_pool = static_cast<const uint16_t*>(k);
+    p.v_pool = static_cast<const uint16_t*>(v);
+    p.k_ids = p.v_ids = nullptr;
+    p.n_pages = int32_t((S + kPage - 1) / kPage);
+    p.n_cached = seq_len;
+    p.S = seq_len;
+    p.Hq = n_q_heads;
+    p.Hkv = n_kv_heads;
+    p.G = n_kv_groups;
+    p.scale_log2 = scale * kLog2e;
+    p.causal = causal != 0;
+    p.page_elems = kPage * D;
+    p.kv_row = D;
+    p.kv_head_stride = S * D;
+    const int64_t q_entry = n_q_heads * S * D, kv_entry = n_kv_heads * S * D;
+    return launch_paged_prefill(p, head_dim, as_stream(stream), PrefillBatch{batch, q_entry, q_entry, kv_entry});
 }

@@ -5,19 +5,24 @@
 // at q_abs = n_cached - S + s and attends keys 0..q_abs (causal, :164-181),
 // kv head = q head / groups (:158).
 //
-// Grid: query tiles of 64 rows x Hq workgroups of 8 waves: the long half of
-// the query tiles from the last down, then the short half from the first up;
-// q heads placed so that those of one kv head share an XCD.
-// Wave w = qb + 4 kh owns query block qb (16 queries) of the tile and key
+// Rows: the S x groups (query, q head) pairs of a kv head, q heads fastest, in
+// row tiles of 64, so a short chunk fills its tiles and the q heads of a kv
+// head share their key tiles.  Grid: row tiles x (batch entry, kv head) pairs,
+// workgroups of 8 waves: the long half of the row tiles from the last down,
+// then the short half from the first up; or, where that would leave the chip
+// idle, row tiles x key splits, merged by a second kernel (prefill_splits).
+// All batch entries go in one launch: two prompts of 1000 tokens (16 q / 8 kv
+// heads of 128) 16.9 us in one launch of 512 workgroups, 29.5 us in two.
+// Wave w = qb + 4 kh owns row block qb (16 rows) of the tile and key
 // half kh (32 keys) of every key tile of 64 tokens (4 pages), so the two key
-// halves of a query block share a SIMD (waves w and w + 4; measured 30.9
+// halves of a row block share a SIMD (waves w and w + 4; measured 30.9
 // against 31.5 us at config 4 and 47.4 against 48.1 us at head_dim 256 with
-// the halves of two query blocks paired instead); the two halves of a query
+// the halves of two row blocks paired instead); the two halves of a row
 // block are merged through LDS at the end.  At
 // head_dim 128 a workgroup holds 64 KB of LDS and at most 128 VGPRs per lane,
 // so two workgroups share a CU (4 waves per SIMD: one workgroup's barrier
 // waits and dependent chains are filled by the other's work); the grid's
-// order puts a long and a short query tile on each CU.  At head_dim 256 (128
+// order puts a long and a short row tile on each CU.  At head_dim 256 (128
 // KB) one workgroup runs per CU.
 // Key tiles are staged in two LDS buffers (one tile in flight while the other
 // is computed), K and V each as [token][dim] rows whose 16-byte chunks are
@@ -50,10 +55,19 @@ namespace genllm {
 namespace {
 
 constexpr int KT = 64;          // keys per tile (4 pages)
-constexpr int QW = 16;          // queries per wave (one 16-column block of O^T)
-constexpr int WAVES = 8;        // query block (4) x key half (2)
-constexpr int QT = 4 * QW;      // queries per query tile
+constexpr int QW = 16;          // rows per wave (one 16-column block of O^T)
+constexpr int WAVES = 8;        // row block (4) x key half (2)
+constexpr int QT = 4 * QW;      // rows per row tile
 constexpr int IDS_BLOCK = 64;   // tiles whose page ids one vector load brings
+constexpr int kMaxPrefillSplits = 32;
+
+// What a launch adds to the attention parameters: batch entries (element
+// strides between them) and the key splits.
+struct PrefillGrid {
+    int64_t q_batch = 0, o_batch = 0, kv_batch = 0;
+    int32_t batch = 1, n_splits = 1;
+    float* partial = nullptr;  // n_splits > 1: o [split][unit][row][D], then {m, l} [split][unit][row]
+};
 
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
@@ -115,23 +129,20 @@ __device__ __forceinline__ void tile_barrier() {
 // (the row's, in lane g = 0; 0 elsewhere, as the hand-over adds the four
 // lanes).  Called only by waves whose tiled state came out NaN or infinite.
 template <int D, bool F16>
-__device__ __forceinline__ void prefill_exact_half(const AttnParams& p, int hq, int q0, int kh, int wave_end,
-                                                   int n_tiles, float* res) {
+__device__ __forceinline__ void prefill_exact_half(const AttnParams& p, const uint16_t* qrow, int64_t kv_off, int s_row,
+                                                   int kh, int wave_end, int t_begin, int t_end, float* res) {
     using E = Elem<F16>;
     constexpr int KS = D / 32, DB = D / 16, KH = KT / 2;
-    const int lane = threadIdx.x & 63, n16 = lane & 15, g = lane >> 4;
-    const int n_cached = p.n_cached, qabs0 = p.n_cached - p.S;
-    const int lim = p.causal ? min(qabs0 + q0 + n16 + 1, n_cached) : n_cached;
-    const int hkv = hq / p.G;
-    const int64_t head_off = int64_t(hkv) * (p.kv_head_stride ? p.kv_head_stride : D);
+    const int g = (threadIdx.x & 63) >> 4;
+    const int n_cached = p.n_cached;
+    const int lim = p.causal ? min(p.n_cached - p.S + s_row + 1, n_cached) : n_cached;
     const bool paged = p.k_ids != nullptr;
-    const uint16_t* const qrow = p.q + int64_t(hq) * p.q_head_stride + int64_t(min(q0 + n16, p.S - 1)) * p.q_tok_stride;
     const float c = fmaxf(p.scale_log2, __FLT_MIN__);
     float m = -INFINITY, l = 0.0f;
     f32x4_t acc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db) acc[db] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int t = 0; t < n_tiles; ++t) {
+    for (int t = t_begin; t < t_end; ++t) {
         for (int j = 0; j < KH; ++j) {
             const int tok = t * KT + KH * kh + j;
             if (tok >= wave_end) break;  // wave-uniform
@@ -142,7 +153,7 @@ __device__ __forceinline__ void prefill_exact_half(const AttnParams& p, int hq, 
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
                 const uint4 qq = *reinterpret_cast<const uint4*>(qrow + 32 * ks + 8 * g);
-                const uint4 kk = *reinterpret_cast<const uint4*>(p.k_pool + head_off + krow + 32 * ks + 8 * g);
+                const uint4 kk = *reinterpret_cast<const uint4*>(p.k_pool + kv_off + krow + 32 * ks + 8 * g);
                 const uint32_t qw[4] = {qq.x, qq.y, qq.z, qq.w}, kw[4] = {kk.x, kk.y, kk.z, kk.w};
 #pragma unroll
                 for (int w2 = 0; w2 < 4; ++w2) {
@@ -160,7 +171,7 @@ __device__ __forceinline__ void prefill_exact_half(const AttnParams& p, int hq, 
             l = vis ? __builtin_fmaf(l, alpha, pk) : l;
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
-                const uint2 u = *reinterpret_cast<const uint2*>(p.v_pool + head_off + vrow + 16 * db + 4 * g);
+                const uint2 u = *reinterpret_cast<const uint2*>(p.v_pool + kv_off + vrow + 16 * db + 4 * g);
                 const float v4[4] = {E::lo(u.x), E::hi(u.x), E::lo(u.y), E::hi(u.y)};
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[db][i] = vis ? __builtin_fmaf(pk, v4[i], acc[db][i] * alpha) : acc[db][i];
@@ -176,8 +187,8 @@ __device__ __forceinline__ void prefill_exact_half(const AttnParams& p, int hq, 
     res[4 * DB + 1] = g == 0 ? l : 0.0f;
 }
 
-template <int D, bool F16>
-__device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
+template <int D, bool F16, bool kSplit>
+__device__ __forceinline__ void prefill_tiles(const AttnParams& p, const PrefillGrid& gr) {
     using E = Elem<F16>;
     constexpr int KS = D / 32, DB = D / 16;
     constexpr int ROWB = D * 2;       // bytes per token row (256 or 512)
@@ -192,39 +203,41 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int qblk = wv & 3, kh = wv >> 2;  // query block, key half (waves w and w + 4 share a SIMD)
+    const int qblk = wv & 3, kh = wv >> 2;  // row block, key half (waves w and w + 4 share a SIMD)
     const int n16 = lane & 15, g = lane >> 4;
-    const int n_qt = (p.S + QT - 1) / QT;
-    const int rank = int(blockIdx.x) / p.Hq;
-    const int slot = int(blockIdx.x) - rank * p.Hq;
-    // Workgroup i runs on XCD i % 8.  With Hq a multiple of 8, slot 8j + x
-    // takes q head x Hq/8 + j, so XCD x holds q heads [x Hq/8, (x+1) Hq/8) and
-    // the q heads of one kv head read its tiles through one L2 (config 4:
-    // FETCH_SIZE 16.2 against 24.2 MiB per launch, the algorithmic q and K/V
-    // bytes against 1.5x; 30.32-30.41 against 30.44-30.56 us, A/B on one box)
-    const int hq = (p.Hq & 7) == 0 ? (slot & 7) * (p.Hq >> 3) + (slot >> 3) : slot;
-    // the first half of the grid runs the query tiles with the most keys, from
-    // the last tile down; the second half the others from the first tile up,
-    // so that workgroups i and i + half the grid -- the two a CU holds when
-    // every workgroup is resident (head_dim 128: 512 workgroups of two per
-    // CU at 16 heads) -- carry n_qt + 1 key tiles between them (A/B at config
-    // 4: 34.5-34.7 against 36.0-36.2 us with the second half running down too)
-    const int half = (n_qt + 1) / 2;
-    const int qt = rank < half ? n_qt - 1 - rank : rank - half;
-    const int hkv = hq / p.G;
+    const int G = p.G, R = p.S * G;  // rows of a kv head: row r is q head r % G of query r / G
+    const int n_rt = (R + QT - 1) / QT;
+    // Workgroup i runs on XCD i % 8: with the (batch entry, kv head) pairs
+    // fastest and 8 kv heads, XCD x holds kv head x and its tiles are read
+    // through one L2 (config 4: FETCH_SIZE 16.2 against 24.2 MiB per launch
+    // with a kv head's rows spread over two XCDs)
+    const int units = gr.batch * p.Hkv;
+    const int rank = int(blockIdx.x) / units;
+    const int unit = int(blockIdx.x) - rank * units;
+    const int bat = unit / p.Hkv, hkv = unit - bat * p.Hkv;
+    // Unsplit: the first half of the grid runs the row tiles with the most
+    // keys, from the last tile down; the second half the others from the first
+    // tile up, so that workgroups i and i + half the grid -- the two a CU holds
+    // when every workgroup is resident (head_dim 128: 512 workgroups of two per
+    // CU at 16 heads) -- carry the same sum of key tiles (A/B at config 4:
+    // 34.5-34.7 against 36.0-36.2 us with the second half running down too).
+    // Split: every workgroup has about the same number of key tiles.
+    const int half = (n_rt + 1) / 2;
+    const int rt = kSplit ? rank / gr.n_splits : rank < half ? n_rt - 1 - rank : rank - half;
+    const int sp = kSplit ? rank - rt * gr.n_splits : 0;
     const int qabs0 = p.n_cached - p.S;
-    const int q0 = qt * QT + qblk * QW;
+    const int q0 = rt * QT + qblk * QW;  // first row of the wave
     const int n_cached = p.n_cached;
 
-    // Q^T operands: lane -> query q0 + n16, dims 32ks + 8g..+7 (a query past
-    // the chunk loads the last row: its column stays finite and is not written)
+    // Q^T operands: lane -> row q0 + n16, dims 32ks + 8g..+7 (a row past the
+    // last one loads the last row: its column stays finite and is not written)
+    const int row = min(q0 + n16, R - 1);
+    const int s_row = row / G;  // the row's query
+    const uint16_t* const qrow = p.q + bat * gr.q_batch + int64_t(hkv * G + (row - s_row * G)) * p.q_head_stride +
+                                 int64_t(s_row) * p.q_tok_stride;
     uint4 qb[KS];  // raw 16-bit elements
-    {
-        const int s = min(q0 + n16, p.S - 1);
-        const uint16_t* qrow = p.q + int64_t(hq) * p.q_head_stride + int64_t(s) * p.q_tok_stride;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) qb[ks] = *reinterpret_cast<const uint4*>(qrow + 32 * ks + 8 * g);
-    }
+    for (int ks = 0; ks < KS; ++ks) qb[ks] = *reinterpret_cast<const uint4*>(qrow + 32 * ks + 8 * g);
     float m = -INFINITY, l = 0.0f;
     // nm = -m (0 while m = -inf); th = the raw score above which the scaled
     // score exceeds m + 8 (-inf while m = -inf)
@@ -233,14 +246,21 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
 #pragma unroll
     for (int db = 0; db < DB; ++db) acc[db] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int wg_last = min(qt * QT + QT, p.S) - 1;
-    const int kv_end = p.causal ? min(qabs0 + wg_last + 1, n_cached) : n_cached;
-    const int n_tiles = (kv_end + KT - 1) / KT;
-    const bool wave_has_rows = q0 < p.S;
-    // keys below wave_lim are visible to every query of the wave, keys at or
-    // past wave_end to none of them
-    const int wave_lim = p.causal ? min(qabs0 + q0 + 1, n_cached) : n_cached;
-    const int wave_end = !wave_has_rows ? 0 : p.causal ? min(qabs0 + min(q0 + QW, p.S), n_cached) : n_cached;
+    const int s_last = (min(rt * QT + QT, R) - 1) / G;  // last query of the workgroup
+    const int kv_last = p.causal ? min(qabs0 + s_last + 1, n_cached) : n_cached;
+    const int n_tiles = (kv_last + KT - 1) / KT;
+    // key tiles [t_begin, t_end) of this workgroup; keys at or past kv_end are
+    // another split's, or no row of the tile sees them
+    const int t_begin = kSplit ? int(int64_t(n_tiles) * sp / gr.n_splits) : 0;
+    const int t_end = kSplit ? int(int64_t(n_tiles) * (sp + 1) / gr.n_splits) : n_tiles;
+    const int kv_end = kSplit ? min(kv_last, t_end * KT) : kv_last;
+    const bool wave_has_rows = q0 < R;
+    // keys below wave_lim are visible to every row of the wave, keys at or
+    // past wave_end to none of them (or not this split's)
+    const int wave_lim = p.causal ? min(qabs0 + q0 / G + 1, n_cached) : n_cached;
+    const int wave_end = !wave_has_rows ? 0
+                         : p.causal     ? min(qabs0 + (min(q0 + QW, R) - 1) / G + 1, kv_end)
+                                        : kv_end;
 
     // ---- staging: wave w < 4 moves page w of each tile, its K rows, then its
     // V rows; waves 4-7 issue no tile loads.  Waves 4-7 share their SIMDs
@@ -254,7 +274,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
     const bool paged = p.k_ids != nullptr;
     const int pg = wv & 3;  // this wave's page of the tile (waves 0-3)
     const bool dma_wave = wv < 4;
-    const int64_t head_off = int64_t(hkv) * (p.kv_head_stride ? p.kv_head_stride : D);
+    const int64_t head_off = bat * gr.kv_batch + int64_t(hkv) * (p.kv_head_stride ? p.kv_head_stride : D);
     const int64_t kv_row = p.kv_row, page_elems = p.page_elems;
     const int kv_row_bytes = int(kv_row) * 2;
     // lane i <- the K (kindx 0) or V (1) id of page pg of tile t0 + i
@@ -311,17 +331,16 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-                const int row = r0 + 16 * kb + n16;
+                const int krow = r0 + 16 * kb + n16;
                 const int pos = 16 * (ks >> 2) + ((4 * (ks & 3) + g) ^ swz(n16));
                 const u32x4_t a = *reinterpret_cast<const __attribute__((address_space(3))) u32x4_t*>(
-                    buf + (row * ROWB + pos * 16));
+                    buf + (krow * ROWB + pos * 16));
                 s[kb] = E::mma32(__builtin_bit_cast(uint4, a), qb[ks], s[kb]);
             }
         after_s();
         if (masked) {
             __asm__ volatile("");  // keep a branch: full tiles carry no selects
-            const int qpos = qabs0 + q0 + n16;
-            const int lim = p.causal ? min(qpos + 1, n_cached) : n_cached;
+            const int lim = p.causal ? min(qabs0 + s_row + 1, n_cached) : n_cached;
             const int rel = lim - tok0 - 4 * g;
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
@@ -380,14 +399,15 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
     // in each of waves 0-3; a tile past the last one has no rows below kv_end and reads
     // as zeros.  Page ids arrive IDS_BLOCK tiles per load; the rare reload
     // drains the loads in flight.
-    int ids0 = paged && dma_wave ? load_ids(0, 0) : 0;
-    int ids1 = paged && dma_wave ? load_ids(0, 1) : 0;
+    const int t_ids = t_begin & ~(IDS_BLOCK - 1);
+    int ids0 = paged && dma_wave ? load_ids(t_ids, 0) : 0;
+    int ids1 = paged && dma_wave ? load_ids(t_ids, 1) : 0;
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // q and ids landed
-    issue_tile(0, ids0, ids1, buf0);
+    issue_tile(t_begin, ids0, ids1, buf0);
     auto step = [&](int t, const lds_char* cur, lds_char* nxt) {
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
         tile_barrier();
-        if (((t + 1) & (IDS_BLOCK - 1)) == 0 && t + 1 < n_tiles) {
+        if (((t + 1) & (IDS_BLOCK - 1)) == 0 && t + 1 < t_end) {
             if (paged && dma_wave) {
                 ids0 = load_ids(t + 1, 0);
                 ids1 = load_ids(t + 1, 1);
@@ -415,7 +435,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
         else
             issue_v();
     };
-    for (int t = 0; t < n_tiles; t += 2) {
+    for (int t = t_begin; t < t_end; t += 2) {
         step(t, buf0, buf1);
         step(t + 1, buf1, buf0);
     }
@@ -438,7 +458,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
             for (int i = 0; i < 4; ++i) tsum += acc[db][i];
         if (__any(!(fabsf(tsum) <= __FLT_MAX__))) {
             float res[DB * 4 + 2];
-            prefill_exact_half<D, F16>(p, hq, q0, kh, wave_end, n_tiles, res);
+            prefill_exact_half<D, F16>(p, qrow, head_off, s_row, kh, wave_end, t_begin, t_end, res);
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -470,10 +490,27 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
     float lt = l * a0 + l1 * a1;
     lt += __shfl_xor(lt, 16);
     lt += __shfl_xor(lt, 32);
+    const int r_out = q0 + n16;
+    if (r_out >= R) return;
+    if constexpr (kSplit) {
+        // partials: o [split][unit][row][D], then {m, l} [split][unit][row]
+        const int64_t at = (int64_t(sp) * units + unit) * R + r_out;
+        float* const po = gr.partial + at * D + 4 * g;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            f32x4_t o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = acc[db][i] * a0 + xch[(db * 4 + i) * 64] * a1;
+            *reinterpret_cast<f32x4_t*>(po + 16 * db) = o;
+        }
+        if (g == 0)
+            *reinterpret_cast<float2*>(gr.partial + int64_t(gr.n_splits) * units * R * D + 2 * at) = make_float2(mt, lt);
+        return;
+    }
     const float inv = 1.0f / lt;
-    const int s = q0 + n16;
-    if (s >= p.S) return;
-    uint16_t* orow = p.out + int64_t(hq) * p.o_head_stride + int64_t(s) * p.o_tok_stride;
+    const int s_out = r_out / G;
+    uint16_t* orow = p.out + bat * gr.o_batch + int64_t(hkv * G + (r_out - s_out * G)) * p.o_head_stride +
+                     int64_t(s_out) * p.o_tok_stride;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
         float o[4];
@@ -495,24 +532,164 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p) {
 // (4 waves per SIMD: at config 4 36.2 us, against 41.9 us for the earlier
 // form of one 128 KB, 196-VGPR workgroup per CU running two query tiles of
 // 2 x 32 queries, A/B on one box); D = 256: 128 KB, one workgroup per CU.
-template <bool F16>
-__global__ __launch_bounds__(WAVES * 64, 2) void paged_prefill_d128_kernel(AttnParams p) { prefill_tiles<128, F16>(p); }
-template <bool F16>
-__global__ __launch_bounds__(WAVES * 64) void paged_prefill_d256_kernel(AttnParams p) { prefill_tiles<256, F16>(p); }
+template <bool F16, bool kSplit>
+__global__ __launch_bounds__(WAVES * 64, 2) void paged_prefill_d128_kernel(AttnParams p, PrefillGrid gr) {
+    prefill_tiles<128, F16, kSplit>(p, gr);
+}
+template <bool F16, bool kSplit>
+__global__ __launch_bounds__(WAVES * 64) void paged_prefill_d256_kernel(AttnParams p, PrefillGrid gr) {
+    prefill_tiles<256, F16, kSplit>(p, gr);
+}
+
+// Merge of the key splits: 4 dims per lane (D / 4 lanes per row), kMergeU
+// splits in flight, with the log-sum-exp rule
+//   M = max m_s, L = sum l_s 2^(m_s - M), O = sum o_s 2^(m_s - M), out = O / L.
+constexpr int kMergeThreads = 256, kMergeU = 8;
+template <int D, bool F16>
+__global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(AttnParams p, PrefillGrid gr) {
+    constexpr int LR = D / 4;
+    const int G = p.G, R = p.S * G, units = gr.batch * p.Hkv;
+    const int64_t rows = int64_t(units) * R;
+    const int64_t at = int64_t(blockIdx.x) * (kMergeThreads / LR) + threadIdx.x / LR;
+    if (at >= rows) return;
+    const int ns = gr.n_splits, d0 = 4 * (threadIdx.x % LR);
+    const float2* const ml = reinterpret_cast<const float2*>(gr.partial + ns * rows * D) + at;
+    const float* const po = gr.partial + at * D + d0;
+    float M = -INFINITY, L = 0.0f;
+    f32x4_t O = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < ns; s0 += kMergeU) {
+        f32x4_t ov[kMergeU];
+        float2 mv[kMergeU];
+#pragma unroll
+        for (int u = 0; u < kMergeU; ++u) {
+            const bool in = s0 + u < ns;
+            const int64_t off = int64_t(in ? s0 + u : s0) * rows;
+            ov[u] = *reinterpret_cast<const f32x4_t*>(po + off * D);
+            mv[u] = ml[off];
+            if (!in) mv[u].x = -INFINITY;
+        }
+        float bm = M;
+#pragma unroll
+        for (int u = 0; u < kMergeU; ++u) bm = fmaxf(bm, mv[u].x);
+        const float a = M == -INFINITY ? 0.0f : exp2_fast(M - bm);
+        L *= a;
+        O *= a;
+#pragma unroll
+        for (int u = 0; u < kMergeU; ++u) {
+            const bool on = mv[u].x != -INFINITY;  // a split that saw no key weighs nothing
+            const float w = on ? exp2_fast(mv[u].x - bm) : 0.0f;
+            L += on ? mv[u].y * w : 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) O[i] += on ? ov[u][i] * w : 0.0f;
+        }
+        M = bm;
+    }
+    const float inv = 1.0f / L;
+    const int unit = int(at / R), r = int(at - int64_t(unit) * R), s = r / G;
+    const int bat = unit / p.Hkv, hkv = unit - bat * p.Hkv;
+    uint16_t* const orow = p.out + bat * gr.o_batch + int64_t(hkv * G + (r - s * G)) * p.o_head_stride +
+                           int64_t(s) * p.o_tok_stride + d0;
+    *reinterpret_cast<uint2*>(orow) = make_uint2(pack2(Elem<F16>::out(O[0] * inv), Elem<F16>::out(O[1] * inv)),
+                                                 pack2(Elem<F16>::out(O[2] * inv), Elem<F16>::out(O[3] * inv)));
+}
+
+template <int D, bool F16>
+int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, hipStream_t stream) {
+    const int64_t rows = int64_t(p.S) * p.G, units = int64_t(gr.batch) * p.Hkv;
+    const dim3 grid(unsigned((rows + QT - 1) / QT * units * gr.n_splits)), block(WAVES * 64);
+    if (gr.n_splits == 1) {
+        if constexpr (D == 128)
+            hipLaunchKernelGGL((paged_prefill_d128_kernel<F16, false>), grid, block, 0, stream, p, gr);
+        else
+            hipLaunchKernelGGL((paged_prefill_d256_kernel<F16, false>), grid, block, 0, stream, p, gr);
+        GENLLM_LAUNCH_CHECK("paged_prefill kernel");
+        return GENLLM_OK;
+    }
+    if constexpr (D == 128)
+        hipLaunchKernelGGL((paged_prefill_d128_kernel<F16, true>), grid, block, 0, stream, p, gr);
+    else
+        hipLaunchKernelGGL((paged_prefill_d256_kernel<F16, true>), grid, block, 0, stream, p, gr);
+    GENLLM_LAUNCH_CHECK("paged_prefill kernel");
+    constexpr int kMergeWgRows = kMergeThreads / (D / 4);
+    hipLaunchKernelGGL((paged_prefill_merge_kernel<D, F16>), dim3(unsigned((rows * units + kMergeWgRows - 1) / kMergeWgRows)),
+                       dim3(kMergeThreads), 0, stream, p, gr);
+    GENLLM_LAUNCH_CHECK("paged_prefill_merge_kernel");
+    return GENLLM_OK;
+}
+
+int resident_workgroups(int head_dim) { return device_cu_count() * (head_dim == 128 ? 2 : 1); }
 
 }  // namespace
 
-int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream) {
+// Every split launch keeps its workgroups resident at once, 64 rows each, so
+// its partials fit this whatever its shape (17 MB at either head_dim).  A
+// cache of up to 4 key tiles is never split.
+size_t prefill_workspace_bytes(int head_dim, int64_t max_tokens) {
+    if ((head_dim != 128 && head_dim != 256) || max_tokens <= 4 * KT) return 0;
+    return size_t(resident_workgroups(head_dim)) * QT * (head_dim + 2) * sizeof(float);
+}
+
+// Key splits of a launch of `rows` rows for each of `units` (batch entry, kv
+// head) pairs: the count with the least estimated time among those whose
+// workgroups are all resident at once, if it beats the unsplit launch by a
+// tenth.  Unsplit, a chunk of few rows leaves
+// most CUs idle while each of its workgroups walks all key tiles in turn.
+// Estimate, in us (fitted to kernel traces on MI355X): a workgroup's longest
+// chain of key tiles at kTileUs each (kTilePairUs where two workgroups share a
+// CU), and for a split launch the hand-over and the merge kernel, kMergeUs plus
+// kMergeUsPerMB of partials written and read back.  Measured, both kernels
+// against the unsplit one (q / kv heads, head_dim, queries at the end of N keys):
+//   32/8, 128,   8 of 8200: 18.8 against 148.6 us (26 splits)
+//   32/8, 128,  64 of 8256: 30.1 against 138.6 us (8)
+//   32/8, 128, 256 of 4096: 35.5 against  65.1 us (4)
+//   32/8, 128, 512 of 8192: 90.2 against 131.6 us (2)
+//   32/8, 128, 512 of 4096: 54.8 against  66.3 us (2), and 52 against 53 us
+//     where the keys are still in the caches: left unsplit, as is 512 of 2048
+//     (36.4 against 35.4 us)
+//   16/8, 128,  64 of 1024: 12.5 against  22.2 us (8)
+//   8/2,  256, 128 of 1128: 18.3 against  29.8 us (6)
+//   8/2,  256,  64 of 8192: 24.7 against 186.2 us (26)
+int prefill_splits(int64_t units, int64_t rows, int n_cached, int head_dim, size_t ws_bytes) {
+    const double kTileUs = head_dim == 128 ? 0.85 : 1.45, kTilePairUs = 1.25, kMergeUs = 6.0, kMergeUsPerMB = 0.46;
+    const int64_t cus = device_cu_count(), wgs = (rows + QT - 1) / QT * units;
+    const int64_t tiles = (int64_t(n_cached) + KT - 1) / KT;
+    const int64_t most = std::min<int64_t>({resident_workgroups(head_dim) / wgs, tiles, kMaxPrefillSplits});
+    int best = 1;
+    double best_us = 0.9 * double(tiles) * kTileUs;
+    for (int64_t ns = 2; ns <= most; ++ns) {
+        const double bytes = double(ns * units * rows) * (head_dim + 2) * sizeof(float);
+        if (bytes > double(ws_bytes)) break;
+        const double us = double((tiles + ns - 1) / ns) * (wgs * ns <= cus ? kTileUs : kTilePairUs) + kMergeUs +
+                          bytes * 1e-6 * kMergeUsPerMB;
+        if (us < best_us) best = int(ns), best_us = us;
+    }
+    return best;
+}
+
+int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream, const PrefillBatch& b, float* ws,
+                         size_t ws_bytes) {
     if (head_dim != 128 && head_dim != 256) return fail(GENLLM_ERR_UNSUPPORTED, "paged prefill: head_dim must be 128 or 256");
-    if (p.S <= 0 || p.n_pages <= 0) return GENLLM_OK;
-    const dim3 grid(unsigned(int64_t((p.S + QT - 1) / QT) * p.Hq)), block(WAVES * 64);
-    if (head_dim == 128)
-        hipLaunchKernelGGL(p.f16 ? paged_prefill_d128_kernel<true> : paged_prefill_d128_kernel<false>, grid, block, 0,
-                           stream, p);
-    else
-        hipLaunchKernelGGL(p.f16 ? paged_prefill_d256_kernel<true> : paged_prefill_d256_kernel<false>, grid, block, 0,
-                           stream, p);
-    GENLLM_LAUNCH_CHECK("paged_prefill kernel");
+    if (p.S <= 0 || p.n_pages <= 0 || b.n <= 0) return GENLLM_OK;
+    const int64_t rows = int64_t(p.S) * p.G;
+    // entries per launch: a grid of at most 2^22 workgroups (HIP takes up to 2^32 threads)
+    const int64_t per = std::max<int64_t>(1, (int64_t(1) << 22) / ((rows + QT - 1) / QT * p.Hkv));
+    for (int64_t b0 = 0; b0 < b.n; b0 += per) {
+        AttnParams pb = p;
+        pb.q += b0 * b.q_stride;
+        pb.out += b0 * b.o_stride;
+        pb.k_pool += b0 * b.kv_stride;
+        pb.v_pool += b0 * b.kv_stride;
+        PrefillGrid gr;
+        gr.batch = int32_t(std::min<int64_t>(per, b.n - b0));
+        gr.q_batch = b.q_stride;
+        gr.o_batch = b.o_stride;
+        gr.kv_batch = b.kv_stride;
+        gr.partial = ws;
+        gr.n_splits = ws ? prefill_splits(int64_t(gr.batch) * p.Hkv, rows, p.n_cached, head_dim, ws_bytes) : 1;
+        const int rc = head_dim == 128 ? (p.f16 ? launch_prefill_d<128, true>(pb, gr, stream) : launch_prefill_d<128, false>(pb, gr, stream))
+                                       : (p.f16 ? launch_prefill_d<256, true>(pb, gr, stream) : launch_prefill_d<256, false>(pb, gr, stream));
+        if (rc) return rc;
+    }
     return GENLLM_OK;
 }
 

@@ -1,0 +1,94 @@
+"""Prefill chunks of the op that are short against the cached keys: the op
+splits their keys over workgroups and a second kernel merges the splits.
+Against the oracle op, at the edges of that path: rows that do not fill a row
+tile of 64 (query, q head) pairs, key counts on and off the 64-key tile, more
+than 64 key tiles (page ids come 64 tiles at a time, and a split may start or
+end inside such a block), fp16, several batch entries, not causal, and NaN and
+infinite inputs in the chunk's own rows.  Tolerances as everywhere (max-abs <=
+2^-7 max|ref| and rel-L2 <= 1e-2 in bf16, 2^-8 and 4e-3 in fp16)."""
+import numpy as np
+import pytest
+import torch
+
+from genllm_amd import paged, synth
+from helpers import assert_attn_close, assert_attn_close_f16, f32, scale_for
+from test_gpu_f16_batch import make
+
+pytestmark = pytest.mark.gpu
+
+
+def chunk(orc, mgr, ref, Hq, Hkv, S, D, seed, f16=False, batch=1, causal=True, plant=None):
+    gen = synth.normal_f16 if f16 else synth.normal_bf16
+    dev = paged.to_device_f16 if f16 else paged.to_device_bf16
+    q = gen(seed, (batch, Hq, S, D))
+    k = gen(seed + 1, (batch, Hkv, S, D)).copy()
+    v = gen(seed + 2, (batch, Hkv, S, D)).copy()
+    if plant:
+        plant(k, v)
+    out = torch.zeros((batch, Hq, S, D), dtype=torch.float16 if f16 else torch.bfloat16, device="cuda")
+    paged.paged_attention(mgr, 0, dev(q), dev(k), dev(v), out, Hq // Hkv, scale_for(D), causal)
+    torch.cuda.synchronize()
+    want, rc = ref.paged_attention(0, q, k, v, Hq // Hkv, scale_for(D), causal, dtype=orc.F16 if f16 else orc.BF16)
+    assert rc == 0
+    return paged.to_host_bits(out), want
+
+
+def cached(orc, Hkv, D, N, S, seed, f16):
+    """A layer holding N - S tokens, written without attending over them."""
+    mgr, ref = make(orc, Hkv, D, (N + 15) // 16 + 3, seed, orc.F16 if f16 else orc.BF16)
+    gen = synth.normal_f16 if f16 else synth.normal_bf16
+    dev = paged.to_device_f16 if f16 else paged.to_device_bf16
+    k, v = gen(seed + 5, (Hkv, N - S, D)), gen(seed + 6, (Hkv, N - S, D))
+    mgr.append_kv_from_pos(0, dev(k), dev(v), 0)
+    ref.append_kv_from_pos(0, k, v, 0)
+    return mgr, ref
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,S,N,f16,batch,causal", [
+    (2, 1, 128, 9, 640, False, 1, True),     # 18 rows: one row tile, mostly empty; 10 whole key tiles
+    (4, 1, 128, 5, 1025, False, 1, True),    # 20 rows, the last key alone in its tile
+    (8, 2, 256, 33, 703, False, 1, True),    # head_dim 256, 132 rows: 3 row tiles, the last of 4 rows
+    (8, 2, 128, 130, 1200, False, 1, True),  # 520 rows: 9 row tiles
+    (4, 2, 128, 20, 4200, False, 1, True),   # 66 key tiles: page ids of two blocks
+    (2, 1, 256, 9, 4100, False, 1, False),   # not causal: every row sees all 65 tiles
+    (3, 3, 128, 40, 1000, True, 1, True),    # fp16, odd head count
+    (4, 2, 128, 17, 900, False, 3, True),    # three batch entries over one cache
+    (16, 1, 128, 2, 2047, False, 1, True),   # 32 rows from two queries
+])
+def test_split_prefill_vs_oracle(orc, Hq, Hkv, D, S, N, f16, batch, causal):
+    mgr, ref = cached(orc, Hkv, D, N, S, 3000 + N, f16)
+    got, want = chunk(orc, mgr, ref, Hq, Hkv, S, D, 4000 + N, f16, batch, causal)
+    label = f"split prefill Hq{Hq} Hkv{Hkv} D{D} S{S} N{N} f16 {f16} batch {batch} causal {causal}"
+    (assert_attn_close_f16 if f16 else assert_attn_close)(got, want, label)
+    mgr.close()
+
+
+@pytest.mark.parametrize("D,S,N", [(128, 24, 1100), (256, 40, 1333)])
+def test_split_prefill_special_values(orc, D, S, N):
+    """A NaN and an infinity in V rows and a NaN in a K row of the chunk's own
+    keys, seen by its later queries only: the same outputs are NaN and infinite
+    as in the oracle (up to the sign of a NaN), the others stay in tolerance."""
+    Hq, Hkv = 4, 2
+
+    def plant(k, v):
+        v[0, 0, S // 2, 3] = 0x7FC0
+        v[0, 0, S // 3, 7] = 0x7F80
+        k[0, 1, S - 4, 11] = 0xFFC0
+
+    mgr, ref = cached(orc, Hkv, D, N, S, 5000 + N, False)
+    got, want = chunk(orc, mgr, ref, Hq, Hkv, S, D, 6000 + N, plant=plant)
+    nf = ~np.isfinite(f32(want))
+    assert nf.any() and np.array_equal(nf, ~np.isfinite(f32(got)))
+    assert np.array_equal(got[nf] & 0x7FFF, want[nf] & 0x7FFF)
+    assert_attn_close(np.where(nf, 0, got).astype(np.uint16), np.where(nf, 0, want).astype(np.uint16), f"special D{D}")
+    mgr.close()
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(3, 4, 2, 70, 128), (5, 2, 1, 1, 256)])
+def test_flash_batch_in_one_launch(orc, B, Hq, Hkv, S, D):
+    """Every batch entry of the non-paged op reads its own q, k and v rows."""
+    q, k, v = (synth.normal_bf16(7000 + i, (B, h, S, D)) for i, h in enumerate((Hq, Hkv, Hkv)))
+    out = torch.zeros((B, Hq, S, D), dtype=torch.bfloat16, device="cuda")
+    paged.flash_attention(*(paged.to_device_bf16(x) for x in (q, k, v)), out, Hq // Hkv, scale_for(D))
+    torch.cuda.synchronize()
+    assert_attn_close(paged.to_host_bits(out), orc.flash_attention(q, k, v, Hq // Hkv, scale_for(D), True), f"flash B{B}")
