@@ -14,7 +14,8 @@
 // All batch entries go in one launch: two prompts of 1000 tokens (16 q / 8 kv
 // heads of 128) 16.9 us in one launch of 512 workgroups, 29.5 us in two.
 // Wave w = qb + 4 kh owns row block qb (16 rows) of the tile and key
-// half kh (32 keys) of every key tile of 64 tokens (4 pages), so the two key
+// part kh (32 keys) of every key tile of 64 tokens (4 pages; 128 tokens and
+// four parts in the 16-wave form, below), so the two key
 // halves of a row block share a SIMD (waves w and w + 4; measured 30.9
 // against 31.5 us at config 4 and 47.4 against 48.1 us at head_dim 256 with
 // the halves of two row blocks paired instead); the two halves of a row
@@ -29,12 +30,12 @@
 // swizzled per 256-byte half: chunk c of row r sits at position
 // 16 (c / 16) + ((c % 16) ^ swz(r % 16)), with swz(r) = 2 ((r % 8) ^ 4 (r / 8))
 // + r / 8.
-// Wave w < 4 moves the K rows, then the V rows of page w of every tile
+// Wave w < 4 (8 in the 16-wave form) moves the K rows, then the V rows of page w of every tile
 // straight from HBM into LDS with 16-byte buffer loads in LDS mode (lane i's
 // 16 bytes land at base + 16 i), so a tile costs no registers, no VALU and no
 // LDS store instructions; one buffer resource per
 // page (base = the page of this kv head, size = the bytes its rows below the
-// key limit span) bounds every load.  Waves 4-7 issue no loads.
+// key limit span) bounds every load.  The other waves issue no loads.
 // Per tile and wave:
 //   S^T = K Q^T  (v_mfma_f32_16x16x32_bf16 x 2 D/32; A = K from LDS: lane l ->
 //        key l%16, dims 32ks+8(l/16)..; B = Q^T held in registers).
@@ -54,10 +55,9 @@ namespace genllm {
 
 namespace {
 
-constexpr int KT = 64;          // keys per tile (4 pages)
+constexpr int KH = 32;          // keys of a tile per wave (the K dimension of the P.V MFMA)
 constexpr int QW = 16;          // rows per wave (one 16-column block of O^T)
-constexpr int WAVES = 8;        // row block (4) x key half (2)
-constexpr int QT = 4 * QW;      // rows per row tile
+constexpr int QT = 4 * QW;      // rows per row tile: 4 row blocks
 constexpr int IDS_BLOCK = 64;   // tiles whose page ids one vector load brings
 constexpr int kMaxPrefillSplits = 32;
 
@@ -122,17 +122,17 @@ __device__ __forceinline__ void tile_barrier() {
     __asm__ volatile("" ::: "memory");
 }
 
-// The key half kh (keys KT t + KH kh .. + KH - 1 of every key tile t) below
+// The key part kh (keys KT t + KH kh .. + KH - 1 of every key tile t) below
 // wave_end, for query q0 + n16 (lane n16 + 16 g), formed the reference's way:
 // per query over the keys it sees, in fp32, one key after another.  res: the
 // O^T values of the lane's dims 16 db + 4 g + i, then m (log2 units) and l
 // (the row's, in lane g = 0; 0 elsewhere, as the hand-over adds the four
 // lanes).  Called only by waves whose tiled state came out NaN or infinite.
-template <int D, bool F16>
-__device__ __forceinline__ void prefill_exact_half(const AttnParams& p, const uint16_t* qrow, int64_t kv_off, int s_row,
+template <int D, bool F16, int KT>
+__device__ __forceinline__ void prefill_exact_part(const AttnParams& p, const uint16_t* qrow, int64_t kv_off, int s_row,
                                                    int kh, int wave_end, int t_begin, int t_end, float* res) {
     using E = Elem<F16>;
-    constexpr int KS = D / 32, DB = D / 16, KH = KT / 2;
+    constexpr int KS = D / 32, DB = D / 16;
     const int g = (threadIdx.x & 63) >> 4;
     const int n_cached = p.n_cached;
     const int lim = p.causal ? min(p.n_cached - p.S + s_row + 1, n_cached) : n_cached;
@@ -187,23 +187,26 @@ __device__ __forceinline__ void prefill_exact_half(const AttnParams& p, const ui
     res[4 * DB + 1] = g == 0 ? l : 0.0f;
 }
 
-template <int D, bool F16, bool kSplit>
+template <int D, bool F16, bool kSplit, int KQ>
 __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const PrefillGrid& gr) {
     using E = Elem<F16>;
     constexpr int KS = D / 32, DB = D / 16;
     constexpr int ROWB = D * 2;       // bytes per token row (256 or 512)
+    constexpr int KT = KQ * KH;       // keys per tile
+    constexpr int KP = KT / kPage;    // pages per tile
     constexpr int TILEB = KT * ROWB;  // bytes of K (or V) per tile
-    constexpr int KH = KT / 2;        // keys of a tile per wave
-    constexpr int XCH = DB * 4 + 2;   // floats per lane handed over at the end: O^T, m, l
-    static_assert(2 * XCH * 64 * 4 <= 2 * TILEB, "two hand-overs fit one buffer");
+    constexpr int XO = DB * 4 * 64;   // floats a wave hands over at the end: O^T, [value][lane]
+    static_assert(KQ == 2 || KQ == 4, "key parts per tile");
+    static_assert(KQ * XO * 4 <= 2 * TILEB, "a buffer holds the hand-overs of KQ waves");
     __shared__ __attribute__((aligned(16))) char lds_b0[2 * TILEB];
     __shared__ __attribute__((aligned(16))) char lds_b1[2 * TILEB];
+    __shared__ float lds_ml[2 * KQ][2][64];  // m and l handed over
     lds_char* const buf0 = (lds_char*)lds_b0;
     lds_char* const buf1 = (lds_char*)lds_b1;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int qblk = wv & 3, kh = wv >> 2;  // row block, key half (waves w and w + 4 share a SIMD)
+    const int qblk = wv & 3, kh = wv >> 2;  // row block, key part (waves w, w + 4, ... share a SIMD)
     const int n16 = lane & 15, g = lane >> 4;
     const int G = p.G, R = p.S * G;  // rows of a kv head: row r is q head r % G of query r / G
     const int n_rt = (R + QT - 1) / QT;
@@ -272,14 +275,14 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     // 30.9 us at config 4, 47.0 against 47.3 at head_dim 256, against one
     // kind per wave over two pages.
     const bool paged = p.k_ids != nullptr;
-    const int pg = wv & 3;  // this wave's page of the tile (waves 0-3)
-    const bool dma_wave = wv < 4;
+    const int pg = wv & (KP - 1);  // this wave's page of the tile (the first KP waves)
+    const bool dma_wave = wv < KP;
     const int64_t head_off = bat * gr.kv_batch + int64_t(hkv) * (p.kv_head_stride ? p.kv_head_stride : D);
     const int64_t kv_row = p.kv_row, page_elems = p.page_elems;
     const int kv_row_bytes = int(kv_row) * 2;
     // lane i <- the K (kindx 0) or V (1) id of page pg of tile t0 + i
     auto load_ids = [&](int t0, int kindx) -> int {
-        const int page = 4 * (t0 + lane) + pg;
+        const int page = KP * (t0 + lane) + pg;
         return page * kPage < kv_end ? (kindx ? p.v_ids : p.k_ids)[page] : 0;
     };
     // instruction e fills rows RPI e .. RPI e + RPI-1 of the page (4 rows of
@@ -396,7 +399,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     // own loads of tile t, meets the other waves (tile t complete in LDS;
     // everybody done with tile t-1), starts tile t+1 into the other buffer,
     // then computes its half of tile t.  Every step issues the same 8 loads
-    // in each of waves 0-3; a tile past the last one has no rows below kv_end and reads
+    // in each loading wave; a tile past the last one has no rows below kv_end and reads
     // as zeros.  Page ids arrive IDS_BLOCK tiles per load; the rare reload
     // drains the loads in flight.
     const int t_ids = t_begin & ~(IDS_BLOCK - 1);
@@ -458,7 +461,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
             for (int i = 0; i < 4; ++i) tsum += acc[db][i];
         if (__any(!(fabsf(tsum) <= __FLT_MAX__))) {
             float res[DB * 4 + 2];
-            prefill_exact_half<D, F16>(p, qrow, head_off, s_row, kh, wave_end, t_begin, t_end, res);
+            prefill_exact_part<D, F16, KT>(p, qrow, head_off, s_row, kh, wave_end, t_begin, t_end, res);
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -468,23 +471,43 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
         }
     }
 
-    // ---- merge the two key halves of each query block: the key-half-1 wave
-    // stores (O^T, m, l) as [value][lane] floats, the key-half-0 wave combines
-    // m = max(m0, m1), O = O0 2^(m0-m) + O1 2^(m1-m), l likewise (a half that
-    // saw no key has m = -inf, weight 0) and writes the output.
+    // ---- merge the key parts of each row block, pair by pair: one wave hands
+    // (O^T, m, l) over through LDS, the other combines m = max(m0, m1), O = O0
+    // 2^(m0-m) + O1 2^(m1-m), l likewise (a part that saw no key has m = -inf,
+    // weight 0).  Four parts: 2 -> 0 and 3 -> 1, then 1 -> 0.
     __syncthreads();  // every wave is done with the tiles
-    lds_float* const xch = (lds_float*)((qblk >> 1) == 0 ? buf0 : buf1) + (qblk & 1) * XCH * 64 + lane;
-    if (kh == 1) {
+    auto slot = [&](int i) { return (lds_float*)(i < KQ ? buf0 : buf1) + (i & (KQ - 1)) * XO + lane; };
+    auto hand_over = [&](int i) {
+        lds_float* const x = slot(i);
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) xch[(db * 4 + i) * 64] = acc[db][i];
-        xch[(DB * 4) * 64] = m;
-        xch[(DB * 4 + 1) * 64] = l;
+            for (int j = 0; j < 4; ++j) x[(db * 4 + j) * 64] = acc[db][j];
+        lds_ml[i][0][lane] = m;
+        lds_ml[i][1][lane] = l;
+    };
+    if constexpr (KQ == 4) {
+        if (kh >= 2) hand_over((kh - 2) * 4 + qblk);
+        __syncthreads();
+        if (kh < 2) {
+            const int i = kh * 4 + qblk;
+            const lds_float* const x = slot(i);
+            const float m1 = lds_ml[i][0][lane], l1 = lds_ml[i][1][lane], mt = fmaxf(m, m1);
+            const float a0 = mt == -INFINITY ? 0.0f : exp2_fast(m - mt), a1 = mt == -INFINITY ? 0.0f : exp2_fast(m1 - mt);
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[db][j] = acc[db][j] * a0 + x[(db * 4 + j) * 64] * a1;
+            m = mt;
+            l = l * a0 + l1 * a1;
+        }
+        __syncthreads();  // the slots are free
     }
+    if (kh == 1) hand_over(qblk);
     __syncthreads();
-    if (kh == 1 || !wave_has_rows) return;
-    const float m1 = xch[(DB * 4) * 64], l1 = xch[(DB * 4 + 1) * 64];
+    if (kh != 0 || !wave_has_rows) return;
+    const lds_float* const xch = slot(qblk);
+    const float m1 = lds_ml[qblk][0][lane], l1 = lds_ml[qblk][1][lane];
     const float mt = fmaxf(m, m1);
     const float a0 = mt == -INFINITY ? 0.0f : exp2_fast(m - mt), a1 = mt == -INFINITY ? 0.0f : exp2_fast(m1 - mt);
     float lt = l * a0 + l1 * a1;
@@ -533,12 +556,25 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
 // form of one 128 KB, 196-VGPR workgroup per CU running two query tiles of
 // 2 x 32 queries, A/B on one box); D = 256: 128 KB, one workgroup per CU.
 template <bool F16, bool kSplit>
-__global__ __launch_bounds__(WAVES * 64, 2) void paged_prefill_d128_kernel(AttnParams p, PrefillGrid gr) {
-    prefill_tiles<128, F16, kSplit>(p, gr);
+__global__ __launch_bounds__(512, 2) void paged_prefill_d128_kernel(AttnParams p, PrefillGrid gr) {
+    prefill_tiles<128, F16, kSplit, 2>(p, gr);
+}
+// 16 waves on 128-key tiles, one workgroup per CU: the same waves per CU as
+// two workgroups of the kernel above, for launches that have only one for
+// each CU.  512 queries (32 q / 8 kv heads) at the end of 1024, 2048, 4096
+// keys: 20.0 against 21.5, 33.6 against 36.3, 58.2 against 66.1 us.  Two
+// independent workgroups stay faster where there are enough (0.63 against
+// 0.87 us per 64 x 64 tile and CU: one barrier holds all 16 waves in step),
+// and below kWideFrom keys the longer start and hand-over cost more than the
+// tiles save (200 of 200: 9.8 against 8.5 us, 40 of 40: 8.7 against 6.3 us).
+constexpr int kWideFrom = 1024;
+template <bool F16>
+__global__ __launch_bounds__(1024) void paged_prefill_d128_wide_kernel(AttnParams p, PrefillGrid gr) {
+    prefill_tiles<128, F16, false, 4>(p, gr);
 }
 template <bool F16, bool kSplit>
-__global__ __launch_bounds__(WAVES * 64) void paged_prefill_d256_kernel(AttnParams p, PrefillGrid gr) {
-    prefill_tiles<256, F16, kSplit>(p, gr);
+__global__ __launch_bounds__(512) void paged_prefill_d256_kernel(AttnParams p, PrefillGrid gr) {
+    prefill_tiles<256, F16, kSplit, 2>(p, gr);
 }
 
 // Merge of the key splits: 4 dims per lane (D / 4 lanes per row), kMergeU
@@ -596,20 +632,22 @@ __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(Attn
 template <int D, bool F16>
 int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, hipStream_t stream) {
     const int64_t rows = int64_t(p.S) * p.G, units = int64_t(gr.batch) * p.Hkv;
-    const dim3 grid(unsigned((rows + QT - 1) / QT * units * gr.n_splits)), block(WAVES * 64);
-    if (gr.n_splits == 1) {
-        if constexpr (D == 128)
-            hipLaunchKernelGGL((paged_prefill_d128_kernel<F16, false>), grid, block, 0, stream, p, gr);
-        else
-            hipLaunchKernelGGL((paged_prefill_d256_kernel<F16, false>), grid, block, 0, stream, p, gr);
-        GENLLM_LAUNCH_CHECK("paged_prefill kernel");
-        return GENLLM_OK;
+    const int64_t wgs = (rows + QT - 1) / QT * units * gr.n_splits;
+    const bool split = gr.n_splits > 1;
+    void (*k)(AttnParams, PrefillGrid);
+    int threads = 512;
+    if constexpr (D == 128) {
+        k = split ? paged_prefill_d128_kernel<F16, true> : paged_prefill_d128_kernel<F16, false>;
+        if (!split && wgs <= device_cu_count() && p.n_cached >= kWideFrom) {
+            k = paged_prefill_d128_wide_kernel<F16>;
+            threads = 1024;
+        }
+    } else {
+        k = split ? paged_prefill_d256_kernel<F16, true> : paged_prefill_d256_kernel<F16, false>;
     }
-    if constexpr (D == 128)
-        hipLaunchKernelGGL((paged_prefill_d128_kernel<F16, true>), grid, block, 0, stream, p, gr);
-    else
-        hipLaunchKernelGGL((paged_prefill_d256_kernel<F16, true>), grid, block, 0, stream, p, gr);
+    hipLaunchKernelGGL(k, dim3(unsigned(wgs)), dim3(threads), 0, stream, p, gr);
     GENLLM_LAUNCH_CHECK("paged_prefill kernel");
+    if (!split) return GENLLM_OK;
     constexpr int kMergeWgRows = kMergeThreads / (D / 4);
     hipLaunchKernelGGL((paged_prefill_merge_kernel<D, F16>), dim3(unsigned((rows * units + kMergeWgRows - 1) / kMergeWgRows)),
                        dim3(kMergeThreads), 0, stream, p, gr);
@@ -625,41 +663,42 @@ int resident_workgroups(int head_dim) { return device_cu_count() * (head_dim == 
 // its partials fit this whatever its shape (17 MB at either head_dim).  A
 // cache of up to 4 key tiles is never split.
 size_t prefill_workspace_bytes(int head_dim, int64_t max_tokens) {
-    if ((head_dim != 128 && head_dim != 256) || max_tokens <= 4 * KT) return 0;
+    if ((head_dim != 128 && head_dim != 256) || max_tokens <= 256) return 0;
     return size_t(resident_workgroups(head_dim)) * QT * (head_dim + 2) * sizeof(float);
 }
 
 // Key splits of a launch of `rows` rows for each of `units` (batch entry, kv
 // head) pairs: the count with the least estimated time among those whose
-// workgroups are all resident at once, if it beats the unsplit launch by a
-// tenth.  Unsplit, a chunk of few rows leaves
+// workgroups are all resident at once.  Unsplit, a chunk of few rows leaves
 // most CUs idle while each of its workgroups walks all key tiles in turn.
 // Estimate, in us (fitted to kernel traces on MI355X): a workgroup's longest
-// chain of key tiles at kTileUs each (kTilePairUs where two workgroups share a
-// CU), and for a split launch the hand-over and the merge kernel, kMergeUs plus
-// kMergeUsPerMB of partials written and read back.  Measured, both kernels
-// against the unsplit one (q / kv heads, head_dim, queries at the end of N keys):
-//   32/8, 128,   8 of 8200: 18.8 against 148.6 us (26 splits)
-//   32/8, 128,  64 of 8256: 30.1 against 138.6 us (8)
-//   32/8, 128, 256 of 4096: 35.5 against  65.1 us (4)
-//   32/8, 128, 512 of 8192: 90.2 against 131.6 us (2)
-//   32/8, 128, 512 of 4096: 54.8 against  66.3 us (2), and 52 against 53 us
-//     where the keys are still in the caches: left unsplit, as is 512 of 2048
-//     (36.4 against 35.4 us)
-//   16/8, 128,  64 of 1024: 12.5 against  22.2 us (8)
-//   8/2,  256, 128 of 1128: 18.3 against  29.8 us (6)
-//   8/2,  256,  64 of 8192: 24.7 against 186.2 us (26)
+// chain of 64-key tiles at kTileUs each (kSplitTileUs in the split kernel, or
+// kPairTileUs where two workgroups share a CU), and for a split launch the
+// hand-over and the merge kernel, kMergeUs plus kMergeUsPerMB of partials
+// written and read back.  Measured, both kernels against one unsplit 8-wave
+// kernel (q / kv heads, head_dim, queries at the end of N keys):
+//   32/8, 128,   8 of 8200: 19.2 against 148.6 us (26 splits)
+//   32/8, 128,  64 of 8256: 30.6 against 138.6 us (8)
+//   32/8, 128, 256 of 4096: 33.7 against  65.1 us (4)
+//   32/8, 128, 512 of 8192: 89.9 against 131.6 us (2; 114.0 with 16 waves)
+//   32/8, 128, 512 of 4096: 54.8 against  66.3 us (2; 58.2 with 16 waves, and
+//     faster than split where the keys are still in L2: left unsplit)
+//   16/8, 128,  64 of 1024: 12.6 against  22.2 us (8)
+//   8/2,  256, 128 of 1128: 18.5 against  29.8 us (6)
+//   8/2,  256,  64 of 8192: 24.0 against 186.2 us (26)
 int prefill_splits(int64_t units, int64_t rows, int n_cached, int head_dim, size_t ws_bytes) {
-    const double kTileUs = head_dim == 128 ? 0.85 : 1.45, kTilePairUs = 1.25, kMergeUs = 6.0, kMergeUsPerMB = 0.46;
+    const bool d128 = head_dim == 128;
+    const double kTileUs = d128 ? 0.8 : 1.45, kSplitTileUs = d128 ? 0.85 : 1.45, kPairTileUs = 1.25;
+    const double kMergeUs = 6.0, kMergeUsPerMB = 0.46;
     const int64_t cus = device_cu_count(), wgs = (rows + QT - 1) / QT * units;
-    const int64_t tiles = (int64_t(n_cached) + KT - 1) / KT;
+    const int64_t tiles = (int64_t(n_cached) + 63) / 64;
     const int64_t most = std::min<int64_t>({resident_workgroups(head_dim) / wgs, tiles, kMaxPrefillSplits});
     int best = 1;
-    double best_us = 0.9 * double(tiles) * kTileUs;
+    double best_us = double(tiles) * kTileUs;
     for (int64_t ns = 2; ns <= most; ++ns) {
         const double bytes = double(ns * units * rows) * (head_dim + 2) * sizeof(float);
         if (bytes > double(ws_bytes)) break;
-        const double us = double((tiles + ns - 1) / ns) * (wgs * ns <= cus ? kTileUs : kTilePairUs) + kMergeUs +
+        const double us = double((tiles + ns - 1) / ns) * (wgs * ns <= cus ? kSplitTileUs : kPairTileUs) + kMergeUs +
                           bytes * 1e-6 * kMergeUsPerMB;
         if (us < best_us) best = int(ns), best_us = us;
     }

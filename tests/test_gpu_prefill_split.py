@@ -12,7 +12,9 @@ import torch
 
 from genllm_amd import paged, synth
 from helpers import assert_attn_close, assert_attn_close_f16, f32, scale_for
+from test_gpu_decode import Context
 from test_gpu_f16_batch import make
+from test_gpu_prefill import run_prefill
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +94,18 @@ def test_flash_batch_in_one_launch(orc, B, Hq, Hkv, S, D):
     paged.flash_attention(*(paged.to_device_bf16(x) for x in (q, k, v)), out, Hq // Hkv, scale_for(D))
     torch.cuda.synchronize()
     assert_attn_close(paged.to_host_bits(out), orc.flash_attention(q, k, v, Hq // Hkv, scale_for(D), True), f"flash B{B}")
+
+
+@pytest.mark.parametrize("Hq,Hkv,S,N,causal", [
+    (4, 2, 33, 1024, True),   # 8 whole 128-key tiles
+    (2, 1, 20, 1025, True),   # the last key alone in its tile
+    (3, 3, 70, 1153, False),  # every key part of the last tile but one is empty
+    (2, 2, 40, 8300, True),   # 65 tiles: page ids of two blocks
+])
+def test_wide_prefill_vs_oracle(orc, Hq, Hkv, S, N, causal):
+    """The stateless entry point never splits; from 1024 keys on a launch with
+    a workgroup or less for each CU runs 16 waves on 128-key tiles."""
+    ctx = Context(orc, Hkv, 128, (N + 15) // 16 + 2, N, 8000 + N, nan_tail=True)
+    q = synth.normal_bf16(8100 + N, (Hq, S, 128))
+    assert_attn_close(run_prefill(ctx, q, causal), ctx.oracle(q, causal), f"wide Hq{Hq} Hkv{Hkv} S{S} N{N} causal {causal}")
+    ctx.close()
