@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 
@@ -19,3 +20,19 @@ def orc():
 
     oracle.build()
     return oracle
+
+
+@pytest.fixture(autouse=True)
+def no_cyclic_gc(request):
+    """No cyclic garbage collection inside a GPU test.  A collection may start
+    at any allocation, and destroying an earlier test's CUDA graph (which waits
+    for the device) while this test captures its own aborts the process: what
+    earlier tests left is collected here, before the test, and the collector
+    stays off until it ends."""
+    if "gpu" not in request.keywords:
+        yield
+        return
+    gc.collect()
+    gc.disable()
+    yield
+    gc.enable()
