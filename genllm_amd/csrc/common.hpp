@@ -129,6 +129,22 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t_ __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t_ __attribute__((ext_vector_type(2)));
 
+// Two fp32 -> packed bf16 for an output, bfloat16_t's constructor
+// (bfloat16.hpp:18-41) for every input: round to nearest even, an fp32
+// subnormal becomes a signed zero, a NaN becomes sign | 0x7F81 (the
+// constructor keeps only "mantissa != 0") -- v_cvt_pk_bf16_f32 plus selects
+// instead of the integer form's branches.
+__device__ __forceinline__ uint32_t bf16_pair_out(float lo, float hi) {
+    const uint32_t nan_lo = ((__float_as_uint(lo) >> 16) & 0x8000u) | 0x7F81u;
+    const uint32_t nan_hi = (__float_as_uint(hi) & 0x80000000u) | 0x7F810000u;
+    const bool lo_nan = lo != lo, hi_nan = hi != hi;
+    lo = fabsf(lo) < __FLT_MIN__ ? __builtin_copysignf(0.0f, lo) : lo;
+    hi = fabsf(hi) < __FLT_MIN__ ? __builtin_copysignf(0.0f, hi) : hi;
+    uint32_t r = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t_{lo, hi}, bf16x2_t_));
+    r = lo_nan ? (r & 0xFFFF0000u) | nan_lo : r;
+    return hi_nan ? (r & 0xFFFFu) | nan_hi : r;
+}
+
 // The 16-bit element type of q, the K/V pools and out: bf16 (F16 = false,
 // every Qwen3 layer) or fp16.  The MFMAs take raw 16-byte (8 elements) or
 // 8-byte (4 elements) operands: both types have the same lane layouts.

@@ -70,15 +70,8 @@ struct PrefillGrid {
 };
 
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) float lds_float;
-
-// two fp32 -> packed bf16 pair, round to nearest even (one v_cvt_pk_bf16_f32)
-__device__ __forceinline__ uint32_t bf16_pair_rne(float lo, float hi) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
-}
 
 // chunk-position swizzle of a 256-byte LDS row, bijective on r % 16.  The
 // K reads (16 rows, one chunk each) hit 16 distinct positions.  A transposing
@@ -93,22 +86,6 @@ __device__ __forceinline__ constexpr int swz(int r) { return (((r & 7) ^ ((r >> 
 __device__ __forceinline__ s16x4_t ds_read_tr(const lds_char* p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         reinterpret_cast<__attribute__((address_space(3))) s16x4_t*>(const_cast<lds_char*>(p)));
-}
-
-// Two fp32 -> packed bf16 for an output, bfloat16_t's constructor
-// (bfloat16.hpp:18-41) for every input: round to nearest even, an fp32
-// subnormal becomes a signed zero, a NaN becomes sign | 0x7F81 (the
-// constructor keeps only "mantissa != 0") -- v_cvt_pk_bf16_f32 plus selects
-// instead of the integer form's branches.
-__device__ __forceinline__ uint32_t bf16_pair_out(float lo, float hi) {
-    const uint32_t nan_lo = ((__float_as_uint(lo) >> 16) & 0x8000u) | 0x7F81u;
-    const uint32_t nan_hi = (__float_as_uint(hi) & 0x80000000u) | 0x7F810000u;
-    const bool lo_nan = lo != lo, hi_nan = hi != hi;
-    lo = fabsf(lo) < __FLT_MIN__ ? __builtin_copysignf(0.0f, lo) : lo;
-    hi = fabsf(hi) < __FLT_MIN__ ? __builtin_copysignf(0.0f, hi) : hi;
-    uint32_t r = bf16_pair_rne(lo, hi);
-    r = lo_nan ? (r & 0xFFFF0000u) | nan_lo : r;
-    return hi_nan ? (r & 0xFFFFu) | nan_hi : r;
 }
 
 // Workgroup barrier for the tile pipeline.  A release fence here would wait
