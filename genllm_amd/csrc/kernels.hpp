@@ -120,7 +120,7 @@ size_t decode_workspace_bytes(int Hq, int Hkv, int S, int D, int n_pages);
 // Decode merge forms (genllm_decode_tuning)
 constexpr int kDecodeMergeKernel = 0, kDecodeMergeFused = 1;
 int set_decode_tuning(int pages_per_split, int merge, int heads_per_wg);
-int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws);
+int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws, size_t* need = nullptr);
 int launch_paged_decode(const AttnParams& p, int head_dim, hipStream_t stream);
 // Batch entries of one prefill launch: element strides between entries (the
 // kv stride is 0 where every entry attends the same cache).

@@ -1219,10 +1219,8 @@ extern "C" int genllm_paged_decode_noalloc(const void* q, int64_t q_head_stride,
         return fail(GENLLM_ERR_INVALID, "paged_decode_noalloc: seq_len * groups must be <= 16");
     void* ws = nullptr;
     if (int rc = scratch_on_device(as_stream(stream), &ws)) return rc;
-    if (int rc = decode_plan(p, head_dim, SIZE_MAX, ws)) return rc;
-    const size_t need = p.n_splits > 1 ? kDecodeCounterBytes + size_t(p.Hkv) * p.n_splits * size_t(p.G * p.S) *
-                                                                 size_t(head_dim + 2) * sizeof(float)
-                                       : 0;
+    size_t need = 0;
+    if (int rc = decode_plan(p, head_dim, SIZE_MAX, ws, &need)) return rc;
     if (need > GENLLM_NOALLOC_SCRATCH_BYTES)
         return fail(GENLLM_ERR_INVALID, "paged_decode_noalloc: this launch needs " + std::to_string(need) +
                                             " bytes of scratch, more than its fixed " +

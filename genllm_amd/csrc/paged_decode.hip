@@ -79,6 +79,15 @@ constexpr int kMaxSplits = 256;
 // more bytes in flight per CU only lengthen the memory queues), 2 at D = 256
 template <int D>
 constexpr int kPagesInFlight = D == 128 ? 1 : 2;
+// Contexts of up to this many pages run in one split, which writes the output
+// itself: one launch and no partials.  Measured, one split against the planned
+// splits and their merge (graph replay over 40 layers, us): 16 q / 8 kv heads
+// of 128, 40 keys 4.1 against 6.4, 128 keys 5.0 against 6.4, 256 keys 6.8
+// against 6.6; 8 / 2 heads of 256, 40 keys 5.2 against 7.2, 80 keys 6.1 against
+// 7.1, 128 keys 7.9 against 7.2.  (Two, three or four pages in flight per wave
+// in that one split: 256 keys 7.5, 7.8, 8.4 us.)
+template <int D>
+constexpr int kOneSplitPages = D == 128 ? 12 : 5;
 constexpr int VT_ROW = kPage + 4;  // LDS V^T row: 16 tokens + pad (bf16 elements)
 constexpr int kNonTemporal = 2;    // buffer-access cache policy bit nt (gfx950: sc0 = 1, nt = 2, sc1 = 16)
 // Cache policy sc1 (agent scope): a store completes at the device's coherence
@@ -857,7 +866,11 @@ int set_decode_tuning(int pages_per_split, int merge, int heads_per_wg) {
 // Heads per workgroup: kMultiHead where the one-head plan reaches
 // kMultiHeadMinPps pages per split (or where forced), for head_dim 128, kv
 // heads in groups of 4 and the merge kernel; else 1.
-int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws) {
+// Short contexts run in one split (kOneSplitPages) unless the split size is
+// forced; the checks of the planned splits are made all the same, and *need is
+// the workspace they ask for.
+int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws, size_t* need_out) {
+    if (need_out) *need_out = 0;
     if (p.G * p.S > kRows) return fail(GENLLM_ERR_INVALID, "paged decode: seq_len * groups must be <= 16");
     DecodeSettings& cfg = decode_settings();
     p.heads_per_wg = 1;
@@ -891,6 +904,14 @@ int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws) {
         if (!ws || ws_bytes < need)
             return fail(GENLLM_ERR_INVALID, "paged decode: workspace too small (need " + std::to_string(need) +
                                                 " bytes, have " + std::to_string(ws_bytes) + ")");
+        if (need_out) *need_out = need;
+        if (cfg.pps.load(std::memory_order_relaxed) <= 0 &&
+            p.n_pages <= (D == 128 ? kOneSplitPages<128> : kOneSplitPages<256>)) {
+            p.pages_per_split = p.n_pages;
+            p.n_splits = 1;
+            p.heads_per_wg = 1;
+            return GENLLM_OK;
+        }
         p.partial = reinterpret_cast<float*>(static_cast<char*>(ws) + kDecodeCounterBytes);
         if (cfg.merge.load(std::memory_order_relaxed) == kDecodeMergeFused) p.counters = static_cast<int32_t*>(ws);
     }

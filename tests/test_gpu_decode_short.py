@@ -1,0 +1,40 @@
+"""Decode over contexts of a few pages: up to kOneSplitPages pages (12 at
+head_dim 128, 5 at 256) one split writes the output itself, above that the
+planned splits and their merge.  Both sides of the line against the oracle,
+and a workspace too small for the planned splits is refused on both."""
+import numpy as np
+import pytest
+
+from genllm_amd import paged, synth
+from genllm_amd._lib import ERR_INVALID, GenllmError
+from helpers import assert_attn_close, scale_for
+from test_gpu_decode import Context
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("Hkv,G,D,S,N,causal", [
+    (8, 4, 128, 1, 192, True),    # 12 whole pages: one split
+    (8, 4, 128, 1, 193, True),    # 13 pages: several splits
+    (1, 16, 128, 1, 33, True),    # 16 rows, the last page holds one key
+    (2, 4, 128, 4, 177, True),    # a chunk of 4 queries across two pages
+    (2, 4, 256, 1, 80, True),     # 5 whole pages at head_dim 256: one split
+    (2, 4, 256, 2, 81, False),    # 6 pages: several splits
+])
+def test_short_decode_vs_oracle(orc, Hkv, G, D, S, N, causal):
+    ctx = Context(orc, Hkv, D, (N + 15) // 16 + 2, N, 8800 + N, nan_tail=True)
+    q = synth.normal_bf16(8900 + N, (Hkv * G, S, D))
+    got, _ = ctx.decode(q, causal=causal)
+    assert_attn_close(got, ctx.oracle(q, causal), f"short decode Hkv{Hkv} G{G} D{D} S{S} N{N}")
+    ctx.close()
+
+
+@pytest.mark.parametrize("N", [100, 300])
+def test_short_decode_keeps_its_workspace_check(N):
+    q = paged.to_device_bf16(synth.normal_bf16(1, (8, 1, 128)))
+    pool = paged.to_device_bf16(np.zeros((20, 16, 2, 128), dtype=np.uint16))
+    ids = paged.to_device_bf16(np.zeros(40, dtype=np.uint16))  # 20 int32 zeros
+    small = paged.to_device_bf16(np.zeros(8, dtype=np.uint16))
+    with pytest.raises(GenllmError) as e:
+        paged.paged_decode(q, q.clone(), pool, pool, ids, ids, (N + 15) // 16, N, 2, scale_for(128), small)
+    assert e.value.code == ERR_INVALID and "workspace too small" in str(e.value)
