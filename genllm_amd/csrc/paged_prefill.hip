@@ -6,7 +6,7 @@
 // kv head = q head / groups (:158).
 //
 // Rows: the S x groups (query, q head) pairs of a kv head, q heads fastest, in
-// row tiles of 64, so a short chunk fills its tiles and the q heads of a kv
+// row tiles of 64 (fewer where CUs would stay idle), so a short chunk fills its tiles and the q heads of a kv
 // head share their key tiles.  Grid: row tiles x (batch entry, kv head) pairs,
 // workgroups of 8 waves: the long half of the row tiles from the last down,
 // then the short half from the first up; or, where that would leave the chip
@@ -61,11 +61,35 @@ constexpr int QT = 4 * QW;      // rows per row tile: 4 row blocks
 constexpr int IDS_BLOCK = 64;   // tiles whose page ids one vector load brings
 constexpr int kMaxPrefillSplits = 32;
 
+// Unsigned division by a divisor known at launch (Granlund and Montgomery,
+// "Division by invariant integers using multiplication", 1994, figure 4.1):
+// exact for every 32-bit dividend, four instructions where the compiler's
+// division takes about thirty (17 queries of 17 keys, 16 q / 8 kv heads: 5.8 ->
+// 5.4 us; 300 of 2000: 21.2 -> 20.3 us).
+struct FastDiv {
+    uint32_t m = 1, s1 = 0, s2 = 0;
+    FastDiv() = default;
+    explicit FastDiv(uint32_t d) {
+        uint32_t l = 0;
+        while (l < 32 && (uint64_t(1) << l) < d) ++l;
+        m = uint32_t(((uint64_t(1) << 32) * ((uint64_t(1) << l) - d)) / d + 1);
+        s1 = l ? 1 : 0;
+        s2 = l ? l - 1 : 0;
+    }
+    __device__ __forceinline__ int operator()(int x) const {
+        const uint32_t t = __umulhi(m, uint32_t(x));
+        return int((t + ((uint32_t(x) - t) >> s1)) >> s2);
+    }
+};
+
 // What a launch adds to the attention parameters: batch entries (element
 // strides between them) and the key splits.
 struct PrefillGrid {
     int64_t q_batch = 0, o_batch = 0, kv_batch = 0;
     int32_t batch = 1, n_splits = 1;
+    int32_t tile_rows = QT;    // rows per row tile: 16, 32 or 64
+    FastDiv by_g, by_units, by_hkv, by_splits;  // groups, batch x kv heads, kv heads, n_splits
+    int32_t n_rt = 0;                           // row tiles of a kv head
     float* partial = nullptr;  // n_splits > 1: o [split][unit][row][D], then {m, l} [split][unit][row]
 };
 
@@ -186,15 +210,16 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     const int qblk = wv & 3, kh = wv >> 2;  // row block, key part (waves w, w + 4, ... share a SIMD)
     const int n16 = lane & 15, g = lane >> 4;
     const int G = p.G, R = p.S * G;  // rows of a kv head: row r is q head r % G of query r / G
-    const int n_rt = (R + QT - 1) / QT;
+    const int tile_rows = gr.tile_rows;
+    const int n_rt = gr.n_rt;
     // Workgroup i runs on XCD i % 8: with the (batch entry, kv head) pairs
     // fastest and 8 kv heads, XCD x holds kv head x and its tiles are read
     // through one L2 (config 4: FETCH_SIZE 16.2 against 24.2 MiB per launch
     // with a kv head's rows spread over two XCDs)
     const int units = gr.batch * p.Hkv;
-    const int rank = int(blockIdx.x) / units;
+    const int rank = gr.by_units(int(blockIdx.x));
     const int unit = int(blockIdx.x) - rank * units;
-    const int bat = unit / p.Hkv, hkv = unit - bat * p.Hkv;
+    const int bat = gr.by_hkv(unit), hkv = unit - bat * p.Hkv;
     // Unsplit: the first half of the grid runs the row tiles with the most
     // keys, from the last tile down; the second half the others from the first
     // tile up, so that workgroups i and i + half the grid -- the two a CU holds
@@ -203,16 +228,16 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     // 34.5-34.7 against 36.0-36.2 us with the second half running down too).
     // Split: every workgroup has about the same number of key tiles.
     const int half = (n_rt + 1) / 2;
-    const int rt = kSplit ? rank / gr.n_splits : rank < half ? n_rt - 1 - rank : rank - half;
+    const int rt = kSplit ? gr.by_splits(rank) : rank < half ? n_rt - 1 - rank : rank - half;
     const int sp = kSplit ? rank - rt * gr.n_splits : 0;
     const int qabs0 = p.n_cached - p.S;
-    const int q0 = rt * QT + qblk * QW;  // first row of the wave
+    const int q0 = rt * tile_rows + qblk * QW;  // first row of the wave
     const int n_cached = p.n_cached;
 
     // Q^T operands: lane -> row q0 + n16, dims 32ks + 8g..+7 (a row past the
     // last one loads the last row: its column stays finite and is not written)
     const int row = min(q0 + n16, R - 1);
-    const int s_row = row / G;  // the row's query
+    const int s_row = gr.by_g(row);  // the row's query
     const uint16_t* const qrow = p.q + bat * gr.q_batch + int64_t(hkv * G + (row - s_row * G)) * p.q_head_stride +
                                  int64_t(s_row) * p.q_tok_stride;
     uint4 qb[KS];  // raw 16-bit elements
@@ -226,20 +251,20 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
 #pragma unroll
     for (int db = 0; db < DB; ++db) acc[db] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int s_last = (min(rt * QT + QT, R) - 1) / G;  // last query of the workgroup
+    const int s_last = gr.by_g(min(rt * tile_rows + tile_rows, R) - 1);  // last query of the workgroup
     const int kv_last = p.causal ? min(qabs0 + s_last + 1, n_cached) : n_cached;
     const int n_tiles = (kv_last + KT - 1) / KT;
     // key tiles [t_begin, t_end) of this workgroup; keys at or past kv_end are
     // another split's, or no row of the tile sees them
-    const int t_begin = kSplit ? int(int64_t(n_tiles) * sp / gr.n_splits) : 0;
-    const int t_end = kSplit ? int(int64_t(n_tiles) * (sp + 1) / gr.n_splits) : n_tiles;
+    const int t_begin = kSplit ? gr.by_splits(n_tiles * sp) : 0;  // n_tiles * 32 < 2^31
+    const int t_end = kSplit ? gr.by_splits(n_tiles * (sp + 1)) : n_tiles;
     const int kv_end = kSplit ? min(kv_last, t_end * KT) : kv_last;
-    const bool wave_has_rows = q0 < R;
+    const bool wave_has_rows = q0 < R && qblk * QW < tile_rows;
     // keys below wave_lim are visible to every row of the wave, keys at or
     // past wave_end to none of them (or not this split's)
-    const int wave_lim = p.causal ? min(qabs0 + q0 / G + 1, n_cached) : n_cached;
+    const int wave_lim = p.causal ? min(qabs0 + gr.by_g(q0) + 1, n_cached) : n_cached;
     const int wave_end = !wave_has_rows ? 0
-                         : p.causal     ? min(qabs0 + (min(q0 + QW, R) - 1) / G + 1, kv_end)
+                         : p.causal     ? min(qabs0 + gr.by_g(min(q0 + QW, R) - 1) + 1, kv_end)
                                         : kv_end;
 
     // ---- staging: wave w < 4 moves page w of each tile, its K rows, then its
@@ -508,7 +533,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
         return;
     }
     const float inv = 1.0f / lt;
-    const int s_out = r_out / G;
+    const int s_out = gr.by_g(r_out);
     uint16_t* orow = p.out + bat * gr.o_batch + int64_t(hkv * G + (r_out - s_out * G)) * p.o_head_stride +
                      int64_t(s_out) * p.o_tok_stride;
 #pragma unroll
@@ -538,13 +563,14 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_d128_kernel(AttnParams p
 }
 // 16 waves on 128-key tiles, one workgroup per CU: the same waves per CU as
 // two workgroups of the kernel above, for launches that have only one for
-// each CU.  512 queries (32 q / 8 kv heads) at the end of 1024, 2048, 4096
-// keys: 20.0 against 21.5, 33.6 against 36.3, 58.2 against 66.1 us.  Two
+// each CU.  512 queries (32 q / 8 kv heads) at the end of 2048, 4096 keys:
+// 33.6 against 36.3, 58.2 against 66.1 us.  Two
 // independent workgroups stay faster where there are enough (0.63 against
 // 0.87 us per 64 x 64 tile and CU: one barrier holds all 16 waves in step),
 // and below kWideFrom keys the longer start and hand-over cost more than the
-// tiles save (200 of 200: 9.8 against 8.5 us, 40 of 40: 8.7 against 6.3 us).
-constexpr int kWideFrom = 1024;
+// tiles save (16 q / 8 kv heads, 1024 of 1024: 16.0 against 15.7 us, 100 of 1100
+// 16.0 against 15.6, 600 of 1500 18.9 against 19.7; 40 of 40: 8.7 against 6.3).
+constexpr int kWideFrom = 1280;
 template <bool F16>
 __global__ __launch_bounds__(1024) void paged_prefill_d128_wide_kernel(AttnParams p, PrefillGrid gr) {
     prefill_tiles<128, F16, false, 4>(p, gr);
@@ -562,12 +588,12 @@ template <int D, bool F16>
 __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(AttnParams p, PrefillGrid gr) {
     constexpr int LR = D / 4;
     const int G = p.G, R = p.S * G, units = gr.batch * p.Hkv;
-    const int64_t rows = int64_t(units) * R;
-    const int64_t at = int64_t(blockIdx.x) * (kMergeThreads / LR) + threadIdx.x / LR;
+    const int rows = units * R;  // at most 64 for each resident workgroup
+    const int at = int(blockIdx.x) * (kMergeThreads / LR) + int(threadIdx.x) / LR;
     if (at >= rows) return;
     const int ns = gr.n_splits, d0 = 4 * (threadIdx.x % LR);
-    const float2* const ml = reinterpret_cast<const float2*>(gr.partial + ns * rows * D) + at;
-    const float* const po = gr.partial + at * D + d0;
+    const float2* const ml = reinterpret_cast<const float2*>(gr.partial + int64_t(ns) * rows * D) + at;
+    const float* const po = gr.partial + int64_t(at) * D + d0;
     float M = -INFINITY, L = 0.0f;
     f32x4_t O = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int s0 = 0; s0 < ns; s0 += kMergeU) {
@@ -598,8 +624,8 @@ __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(Attn
         M = bm;
     }
     const float inv = 1.0f / L;
-    const int unit = int(at / R), r = int(at - int64_t(unit) * R), s = r / G;
-    const int bat = unit / p.Hkv, hkv = unit - bat * p.Hkv;
+    const int unit = at / R, r = at - unit * R, s = gr.by_g(r);
+    const int bat = gr.by_hkv(unit), hkv = unit - bat * p.Hkv;
     uint16_t* const orow = p.out + bat * gr.o_batch + int64_t(hkv * G + (r - s * G)) * p.o_head_stride +
                            int64_t(s) * p.o_tok_stride + d0;
     *reinterpret_cast<uint2*>(orow) = make_uint2(pack2(Elem<F16>::out(O[0] * inv), Elem<F16>::out(O[1] * inv)),
@@ -609,7 +635,7 @@ __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(Attn
 template <int D, bool F16>
 int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, hipStream_t stream) {
     const int64_t rows = int64_t(p.S) * p.G, units = int64_t(gr.batch) * p.Hkv;
-    const int64_t wgs = (rows + QT - 1) / QT * units * gr.n_splits;
+    const int64_t wgs = gr.n_rt * units * gr.n_splits;
     const bool split = gr.n_splits > 1;
     void (*k)(AttnParams, PrefillGrid);
     int threads = 512;
@@ -702,6 +728,19 @@ int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream, 
         gr.kv_batch = b.kv_stride;
         gr.partial = ws;
         gr.n_splits = ws ? prefill_splits(int64_t(gr.batch) * p.Hkv, rows, p.n_cached, head_dim, ws_bytes) : 1;
+        // Where CUs would stay idle, smaller row tiles spread the rows over more
+        // of them, fewer row blocks each (tiles of 16, 32 and 64 rows, us: 16 q
+        // / 8 kv heads, 100 of 700 11.4, 11.5, 11.8; 500 of 1030 15.1, 15.3,
+        // 15.6; 64 of 4000 37.5, 38.1, 39.0).
+        if (gr.n_splits == 1) {
+            const int64_t cus = device_cu_count(), units = int64_t(gr.batch) * p.Hkv;
+            for (int r = QT / 2; r >= QW && (rows + r - 1) / r * units <= cus; r /= 2) gr.tile_rows = r;
+        }
+        gr.n_rt = int32_t((rows + gr.tile_rows - 1) / gr.tile_rows);
+        gr.by_g = FastDiv(uint32_t(p.G));
+        gr.by_units = FastDiv(uint32_t(gr.batch * p.Hkv));
+        gr.by_hkv = FastDiv(uint32_t(p.Hkv));
+        gr.by_splits = FastDiv(uint32_t(gr.n_splits));
         const int rc = head_dim == 128 ? (p.f16 ? launch_prefill_d<128, true>(pb, gr, stream) : launch_prefill_d<128, false>(pb, gr, stream))
                                        : (p.f16 ? launch_prefill_d<256, true>(pb, gr, stream) : launch_prefill_d<256, false>(pb, gr, stream));
         if (rc) return rc;

@@ -97,15 +97,29 @@ def test_flash_batch_in_one_launch(orc, B, Hq, Hkv, S, D):
 
 
 @pytest.mark.parametrize("Hq,Hkv,S,N,causal", [
-    (4, 2, 33, 1024, True),   # 8 whole 128-key tiles
-    (2, 1, 20, 1025, True),   # the last key alone in its tile
-    (3, 3, 70, 1153, False),  # every key part of the last tile but one is empty
+    (4, 2, 33, 1280, True),   # 10 whole 128-key tiles
+    (2, 1, 20, 1281, True),   # the last key alone in its tile
+    (3, 3, 70, 1409, False),  # every key part of the last tile but one is empty
     (2, 2, 40, 8300, True),   # 65 tiles: page ids of two blocks
 ])
 def test_wide_prefill_vs_oracle(orc, Hq, Hkv, S, N, causal):
-    """The stateless entry point never splits; from 1024 keys on a launch with
+    """The stateless entry point never splits; from 1280 keys on a launch with
     a workgroup or less for each CU runs 16 waves on 128-key tiles."""
     ctx = Context(orc, Hkv, 128, (N + 15) // 16 + 2, N, 8000 + N, nan_tail=True)
     q = synth.normal_bf16(8100 + N, (Hq, S, 128))
     assert_attn_close(run_prefill(ctx, q, causal), ctx.oracle(q, causal), f"wide Hq{Hq} Hkv{Hkv} S{S} N{N} causal {causal}")
+    ctx.close()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,S,N,causal", [
+    (4, 4, 128, 17, 17, True),     # 17 rows: two tiles of 16, the second with one row
+    (6, 2, 128, 27, 100, True),    # three q heads per kv head: 81 rows in tiles of 16
+    (64, 32, 128, 80, 100, True),  # tiles of 32 rows: 16 would take more than a workgroup per CU
+    (8, 2, 256, 45, 300, False),   # head_dim 256
+])
+def test_small_row_tiles_vs_oracle(orc, Hq, Hkv, D, S, N, causal):
+    """Launches that leave CUs idle take row tiles of 16 or 32 rows."""
+    ctx = Context(orc, Hkv, D, (N + 15) // 16 + 2, N, 8200 + N + S, nan_tail=True)
+    q = synth.normal_bf16(8300 + N, (Hq, S, D))
+    assert_attn_close(run_prefill(ctx, q, causal), ctx.oracle(q, causal), f"row tiles Hq{Hq} Hkv{Hkv} D{D} S{S} N{N}")
     ctx.close()
