@@ -137,4 +137,5 @@ def check(rc: int):
 
 
 def call(name: str, *args):
-    return check(getattr(lib(), name)(*args))
+    rc = getattr(_lib or lib(), name)(*args)
+    return rc if rc == OK else check(rc)
