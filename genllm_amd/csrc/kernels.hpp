@@ -131,8 +131,14 @@ struct PrefillBatch {
 // ws (may be null: no launch is split): scratch for the partials of a
 // key-split launch, prefill_workspace_bytes for the most keys a call may have.
 size_t prefill_workspace_bytes(int head_dim, int64_t max_tokens);
+// append (may be null): the op's append, in the same launch or one before it:
+// the S tokens k_new / v_new of p go to positions new_from .. of the pages.
+struct PrefillAppend {
+    int32_t max_blocks = INT32_MAX;  // ids outside [0, max_blocks) are never written through
+    AppendTableUpdate upd;           // pages opened by this call
+};
 int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream, const PrefillBatch& b = {},
-                         float* ws = nullptr, size_t ws_bytes = 0);
+                         float* ws = nullptr, size_t ws_bytes = 0, const PrefillAppend* append = nullptr);
 
 int launch_rms_norm(uint16_t* out, const uint16_t* x, const float* w, int64_t rows, int hidden, float eps,
                     hipStream_t stream);

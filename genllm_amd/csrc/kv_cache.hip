@@ -359,9 +359,9 @@ int prepare_attention(AttnParams& p, int head_dim, genllm_kv* kv) {
 }
 
 int launch_attention(const AttnParams& p, const LayerState& s, int head_dim, hipStream_t stream,
-                     const PrefillBatch& batch = {}) {
+                     const PrefillBatch& batch = {}, const PrefillAppend* append = nullptr) {
     if (p.G * p.S <= 16) return launch_paged_decode(p, head_dim, stream);
-    return launch_paged_prefill(p, head_dim, stream, batch, s.prefill_ws, s.prefill_ws_bytes);
+    return launch_paged_prefill(p, head_dim, stream, batch, s.prefill_ws, s.prefill_ws_bytes, append);
 }
 
 }  // namespace
@@ -703,50 +703,32 @@ extern "C" int genllm_paged_attention(genllm_kv* kv, int32_t layer, const void* 
     if (int rc = prepare_attention(p, head_dim, kv)) return rc;
 
     // 1. append (append_kv_from_tensor, attention.cpp:146): head-major [Hkv][S][D].
-    // Short chunks (the decode kernel's range) append inside the attention
-    // kernel itself: the wave that reads a page takes the new rows from k/v and
-    // writes them to their slots, so no separate launch is needed.
-    AppendParams ap;
+    // The attention kernels do it themselves, taking the new rows from k/v and
+    // writing them to their slots: in short chunks (the decode kernel's range)
+    // the wave that reads a page; in longer ones every workgroup a share, or,
+    // where that would cost more than it saves, a launch before the attention.
+    PrefillAppend pa;
     AppendUndo& undo = t_undo;
-    if (int rc = append_pages(kv, *s, seq_len, st, &ap.upd, &undo)) return rc;
-    ap.k = static_cast<const uint16_t*>(k);
-    ap.v = static_cast<const uint16_t*>(v);
-    ap.k_tok_stride = ap.v_tok_stride = head_dim;
-    ap.k_head_stride = ap.v_head_stride = int64_t(seq_len) * head_dim;
-    ap.S = seq_len;
-    ap.Hkv = n_kv_heads;
-    ap.pos0 = pos0;
-    ap.nkv_tasks = (n_kv_heads + 7) / 8;
-    ap.k_pool = s->k_base;
-    ap.v_pool = s->v_base;
-    ap.page_elems = int64_t(kPage) * n_kv_heads * head_dim;
-    ap.k_ids = s->d_k_ids;
-    ap.v_ids = s->d_v_ids;
-    ap.max_blocks = s->max_blocks;
-    if (!fuse) {
-        if (int rc = launch_kv_append(ap, head_dim, st)) {
-            undo_append(*s, undo);
-            return rc;
-        }
-    }
+    if (int rc = append_pages(kv, *s, seq_len, st, &pa.upd, &undo)) return rc;
+    pa.max_blocks = s->max_blocks;
 
     // 2. attend over all cached tokens
+    fuse_append(p, *s, k, v, seq_len, head_dim, pos0);
     if (fuse) {
-        fuse_append(p, *s, k, v, seq_len, head_dim, pos0);
         // seq_len <= 16 opens at most 2 pages, which fit the launch arguments
-        // (append_pages put them in ap.upd, as it holds up to 256)
+        // (append_pages put them in pa.upd, as it holds up to 256)
         static_assert(sizeof(p.upd.k) / sizeof(int32_t) >= 2, "decode step opens up to 2 pages");
-        p.upd.first = ap.upd.first;
-        p.upd.count = ap.upd.count;
-        for (int32_t i = 0; i < ap.upd.count; ++i) {
-            p.upd.k[i] = ap.upd.k[i];
-            p.upd.v[i] = ap.upd.v[i];
+        p.upd.first = pa.upd.first;
+        p.upd.count = pa.upd.count;
+        for (int32_t i = 0; i < pa.upd.count; ++i) {
+            p.upd.k[i] = pa.upd.k[i];
+            p.upd.v[i] = pa.upd.v[i];
         }
     }
     // Longer chunks take every batch entry in one launch.
     const int64_t entry = int64_t(n_q_heads) * seq_len * head_dim;
-    if (int rc = launch_attention(p, *s, head_dim, st, PrefillBatch{batch, entry, entry, 0})) {
-        if (fuse) undo_append(*s, undo);  // nothing ran: the fused append is part of this launch
+    if (int rc = launch_attention(p, *s, head_dim, st, PrefillBatch{batch, entry, entry, 0}, &pa)) {
+        undo_append(*s, undo);  // the append is part of the launch that failed
         return rc;
     }
     // 3. batch entries after the first attend over the same cache

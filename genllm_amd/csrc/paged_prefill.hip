@@ -48,6 +48,9 @@
 //        own query column, so the rescale by 2^(m_old-m_new) stays lane-local.
 // Causal masking is applied only to the key halves that reach past the first
 // query of the wave (the diagonal) or past the cache end.
+#include <climits>
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -97,6 +100,10 @@ typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) float lds_float;
 
+struct NoAppend {};
+template <bool kNew>
+using AppendArg = std::conditional_t<kNew, PrefillAppend, NoAppend>;
+
 // chunk-position swizzle of a 256-byte LDS row, bijective on r % 16.  The
 // K reads (16 rows, one chunk each) hit 16 distinct positions.  A transposing
 // V read takes 32 bytes (one chunk pair) of each of 16 rows, and the LDS
@@ -130,7 +137,7 @@ __device__ __forceinline__ void tile_barrier() {
 // (the row's, in lane g = 0; 0 elsewhere, as the hand-over adds the four
 // lanes).  Called only by waves whose tiled state came out NaN or infinite.
 template <int D, bool F16, int KT>
-__device__ __forceinline__ void prefill_exact_part(const AttnParams& p, const uint16_t* qrow, int64_t kv_off, int s_row,
+__device__ __forceinline__ void prefill_exact_part(const AttnParams& p, const uint16_t* qrow, int64_t kv_off, int hkv, int s_row,
                                                    int kh, int wave_end, int t_begin, int t_end, float* res) {
     using E = Elem<F16>;
     constexpr int KS = D / 32, DB = D / 16;
@@ -148,13 +155,20 @@ __device__ __forceinline__ void prefill_exact_part(const AttnParams& p, const ui
             const int tok = t * KT + KH * kh + j;
             if (tok >= wave_end) break;  // wave-uniform
             const int64_t in_page = int64_t(tok % kPage) * p.kv_row;
-            const int64_t krow = paged ? int64_t(p.k_ids[tok / kPage]) * p.page_elems + in_page : int64_t(tok) * p.kv_row;
-            const int64_t vrow = paged ? int64_t(p.v_ids[tok / kPage]) * p.page_elems + in_page : int64_t(tok) * p.kv_row;
+            const uint16_t *krow, *vrow;
+            if (tok >= p.new_from) {  // appended by this call: its pages may not be written yet
+                const int64_t at = hkv * p.new_head_stride + int64_t(tok - p.new_from) * p.new_tok_stride;
+                krow = p.k_new + at;
+                vrow = p.v_new + at;
+            } else {
+                krow = p.k_pool + kv_off + (paged ? int64_t(p.k_ids[tok / kPage]) * p.page_elems + in_page : int64_t(tok) * p.kv_row);
+                vrow = p.v_pool + kv_off + (paged ? int64_t(p.v_ids[tok / kPage]) * p.page_elems + in_page : int64_t(tok) * p.kv_row);
+            }
             float sp = 0.0f;  // this lane's dims 32 ks + 8 g .. + 7, then the row's four lanes
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
                 const uint4 qq = *reinterpret_cast<const uint4*>(qrow + 32 * ks + 8 * g);
-                const uint4 kk = *reinterpret_cast<const uint4*>(p.k_pool + kv_off + krow + 32 * ks + 8 * g);
+                const uint4 kk = *reinterpret_cast<const uint4*>(krow + 32 * ks + 8 * g);
                 const uint32_t qw[4] = {qq.x, qq.y, qq.z, qq.w}, kw[4] = {kk.x, kk.y, kk.z, kk.w};
 #pragma unroll
                 for (int w2 = 0; w2 < 4; ++w2) {
@@ -172,7 +186,7 @@ __device__ __forceinline__ void prefill_exact_part(const AttnParams& p, const ui
             l = vis ? __builtin_fmaf(l, alpha, pk) : l;
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
-                const uint2 u = *reinterpret_cast<const uint2*>(p.v_pool + kv_off + vrow + 16 * db + 4 * g);
+                const uint2 u = *reinterpret_cast<const uint2*>(vrow + 16 * db + 4 * g);
                 const float v4[4] = {E::lo(u.x), E::hi(u.x), E::lo(u.y), E::hi(u.y)};
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[db][i] = vis ? __builtin_fmaf(pk, v4[i], acc[db][i] * alpha) : acc[db][i];
@@ -188,7 +202,71 @@ __device__ __forceinline__ void prefill_exact_part(const AttnParams& p, const ui
     res[4 * DB + 1] = g == 0 ? l : 0.0f;
 }
 
-template <int D, bool F16, bool kSplit, int KQ>
+// The launch arguments of a kernel that appends, as they lie in its argument
+// block.  late_args() reads them where they are used: after the tile loop, or
+// in the one step that patches a page.  Taken from the kernel's parameters
+// they were held in scalar registers through the loop, which spilled 20-50 of
+// them (a 512-token chunk of 8192 keys: 101.0 -> 98.0 us).
+struct AppendKernelArgs {
+    AttnParams p;
+    PrefillGrid gr;
+    PrefillAppend pa;
+};
+__device__ __forceinline__ const AppendKernelArgs& late_args() {
+    typedef const __attribute__((address_space(4))) AppendKernelArgs args_t;
+    args_t* a = (args_t*)__builtin_amdgcn_kernarg_segment_ptr();
+    __asm__ volatile("" : "+s"(a));
+    return *(const AppendKernelArgs*)a;
+}
+
+// The op's append, inside the attention launch: the chunk's K and V rows
+// ([Hkv][S][D]) copied to their page slots bit for bit, 16 bytes per thread and
+// step, kCopy steps in flight; workgroup 0 also writes the ids of the pages
+// opened by this call into the device table.  The attention reads the chunk's
+// rows from k_new / v_new, so nothing waits for these stores; the waves that
+// have handed their state over run it while the others write the output (at
+// the start of the kernel it cost every workgroup 2.5 us).  tid of n_threads:
+// the thread among those of the workgroup that take part.
+constexpr int kCopy = 4;
+template <int D>
+__device__ __forceinline__ void append_chunk(int tid, int n_threads) {
+    const AppendKernelArgs& a = late_args();
+    const AttnParams& p = a.p;
+    const PrefillGrid& gr = a.gr;
+    const PrefillAppend& pa = a.pa;
+    constexpr int CH = D / 8;  // 16-byte chunks per row
+    const int half = p.S * p.Hkv * CH;
+    const int64_t step = int64_t(gridDim.x) * n_threads;
+    if (blockIdx.x == 0)
+        for (int i = tid; i < pa.upd.count; i += n_threads) {
+            p.k_ids_w[pa.upd.first + i] = pa.upd.k[i];
+            p.v_ids_w[pa.upd.first + i] = pa.upd.v[i];
+        }
+    for (int64_t i0 = int64_t(blockIdx.x) * n_threads + tid; i0 < 2 * int64_t(half); i0 += kCopy * step) {
+        uint4 x[kCopy];
+        uint16_t* dst[kCopy];
+#pragma unroll
+        for (int u = 0; u < kCopy; ++u) {
+            const int64_t i = i0 + u * step;
+            dst[u] = nullptr;
+            if (i < 2 * int64_t(half)) {
+                const bool v = i >= half;
+                const int j = int(v ? i - half : i), row = j / CH, c = j % CH;
+                const int t = gr.by_hkv(row), h = row - t * p.Hkv, pos = p.new_from + t;
+                const int rel = pos / kPage - pa.upd.first;
+                const int id = rel >= 0 && rel < pa.upd.count ? (v ? pa.upd.v : pa.upd.k)[rel] : (v ? p.v_ids : p.k_ids)[pos / kPage];
+                x[u] = *reinterpret_cast<const uint4*>((v ? p.v_new : p.k_new) + h * p.new_head_stride + t * p.new_tok_stride + 8 * c);
+                if (id >= 0 && id < pa.max_blocks)
+                    dst[u] = (v ? p.v_pool_w : p.k_pool_w) + id * p.page_elems + (pos % kPage) * p.kv_row + h * D + 8 * c;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kCopy; ++u)
+            if (dst[u]) *reinterpret_cast<uint4*>(dst[u]) = x[u];
+    }
+}
+
+template <int D, bool F16, bool kSplit, int KQ, bool kNew>
 __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const PrefillGrid& gr) {
     using E = Elem<F16>;
     constexpr int KS = D / 32, DB = D / 16;
@@ -285,7 +363,8 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     // lane i <- the K (kindx 0) or V (1) id of page pg of tile t0 + i
     auto load_ids = [&](int t0, int kindx) -> int {
         const int page = KP * (t0 + lane) + pg;
-        return page * kPage < kv_end ? (kindx ? p.v_ids : p.k_ids)[page] : 0;
+        const int end = kNew ? min(kv_end, p.new_from) : kv_end;  // pages that hold earlier tokens
+        return page * kPage < end ? (kindx ? p.v_ids : p.k_ids)[page] : 0;
     };
     // instruction e fills rows RPI e .. RPI e + RPI-1 of the page (4 rows of
     // 256 B at D = 128, 2 of 512 B at D = 256): lane -> row RPI e + lane/LPR,
@@ -302,24 +381,62 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     // The buffer resource of a page spans exactly its rows below kv_end, so
     // rows past the causal limit, the cache end or the table read as zeros:
     // their keys are masked and their zero values meet zero probabilities.
-    auto issue_page = [&](int t, int ids, lds_char* buf, int kindx) {  // K (0) or V (1) rows of page pg of tile t
-        const uint16_t* const src = (kindx ? p.v_pool : p.k_pool) + head_off;
+    // kNew: pages that hold only tokens of this call's chunk are read from its
+    // own rows, which follow each other (ROWB bytes apart); of the page where
+    // the chunk starts only the earlier rows are loaded here (patch_page).
+    const int new_from = kNew ? __builtin_amdgcn_readfirstlane(p.new_from) : INT_MAX;
+    const uint16_t* const k_chunk = kNew ? p.k_new + hkv * p.new_head_stride - int64_t(new_from) * D : nullptr;
+    const uint16_t* const v_chunk = kNew ? p.v_new + hkv * p.new_head_stride - int64_t(new_from) * D : nullptr;
+    // kAny: the page may hold tokens of the chunk.
+    auto issue_page = [&](auto any, int t, int ids, lds_char* buf, int kindx) {  // K (0) or V (1) rows of page pg of tile t
+        constexpr bool kAny = decltype(any)::value;
+        const uint16_t* src = (kindx ? p.v_pool : p.k_pool) + head_off;
         const int tok_page = t * KT + kPage * pg;
-        const int valid = min(max(kv_end - tok_page, 0), kPage);
-        const uint32_t span = uint32_t(__builtin_amdgcn_readfirstlane(valid > 0 ? (valid - 1) * kv_row_bytes + ROWB : 0));
-        const int64_t base = paged ? int64_t(__builtin_amdgcn_readlane(ids, t & (IDS_BLOCK - 1))) * page_elems
-                                   : int64_t(tok_page) * kv_row;
+        int valid = min(max(kv_end - tok_page, 0), kPage);
+        int64_t base = paged ? int64_t(__builtin_amdgcn_readlane(ids, t & (IDS_BLOCK - 1))) * page_elems
+                             : int64_t(tok_page) * kv_row;
+        int row_bytes = kv_row_bytes, less = 0;
+        if constexpr (kAny) {
+            const int ahead = tok_page - new_from;
+            const bool fresh = ahead >= 0;
+            src = fresh ? (kindx ? v_chunk : k_chunk) : src;
+            base = fresh ? int64_t(tok_page) * D : base;
+            row_bytes = fresh ? ROWB : kv_row_bytes;
+            valid = fresh ? valid : min(valid, -ahead);
+            less = kv_row_bytes - row_bytes;
+        }
+        const uint32_t span = uint32_t(__builtin_amdgcn_readfirstlane(valid > 0 ? (valid - 1) * row_bytes + ROWB : 0));
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(src + base), 0, span, kBufferFlags);
+        const uint32_t lane_less = kAny ? uint32_t(lane / LPR) * uint32_t(less) : 0;
 #pragma unroll
         for (int e = 0; e < NI; ++e)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 r, (__attribute__((address_space(3))) void*)(buf + (kindx * TILEB + pg * (kPage * ROWB) + e * 1024)), 16,
-                dma_off[e], 0, 0, 0);
+                kAny ? dma_off[e] - lane_less - uint32_t(RPI * e) * uint32_t(less) : dma_off[e], 0, 0, 0);
     };
-    auto issue_tile = [&](int t, int ids0, int ids1, lds_char* buf) {  // ids0, ids1: K and V ids of page pg
+    // The chunk's rows of the page where it starts inside a page, into the
+    // landed tile (the loads above left zeros there).
+    auto patch_page = [&](lds_char* buf) {
+        const AttnParams& p = late_args().p;
+        const int tok_page = new_from & ~(kPage - 1), cut = new_from - tok_page;
+        const int valid = min(max(kv_end - tok_page, 0), kPage);
+#pragma clang loop unroll(disable)
+        for (int kindx = 0; kindx < 2; ++kindx)
+#pragma clang loop unroll(disable)
+            for (int e = 0; e < NI; ++e) {
+                const int prow = RPI * e + lane / LPR, pos = lane % LPR;
+                const int chunk = 16 * (pos >> 4) + ((pos & 15) ^ swz(prow));
+                if (prow < cut || prow >= valid) continue;
+                const u32x4_t x = *reinterpret_cast<const u32x4_t*>((kindx ? p.v_new : p.k_new) + hkv * p.new_head_stride + int64_t(prow - cut) * D + 8 * chunk);
+                *reinterpret_cast<__attribute__((address_space(3))) u32x4_t*>(
+                    buf + (kindx * TILEB + pg * (kPage * ROWB) + e * 1024 + 16 * lane)) = x;
+            }
+        __builtin_amdgcn_s_waitcnt(0);
+    };
+    auto issue_tile = [&](auto any, int t, int ids0, int ids1, lds_char* buf) {  // ids0, ids1: K and V ids of page pg
         if (dma_wave) {
-            issue_page(t, ids0, buf, 0);
-            issue_page(t, ids1, buf, 1);
+            issue_page(any, t, ids0, buf, 0);
+            issue_page(any, t, ids1, buf, 1);
         }
     };
 
@@ -408,9 +525,13 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     int ids0 = paged && dma_wave ? load_ids(t_ids, 0) : 0;
     int ids1 = paged && dma_wave ? load_ids(t_ids, 1) : 0;
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // q and ids landed
-    issue_tile(t_begin, ids0, ids1, buf0);
-    auto step = [&](int t, const lds_char* cur, lds_char* nxt) {
+    issue_tile(std::bool_constant<kNew>{}, t_begin, ids0, ids1, buf0);
+    auto step = [&](auto any, int t, lds_char* cur, lds_char* nxt) {
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+        if constexpr (decltype(any)::value) {
+            const bool mixed = (new_from & (kPage - 1)) && new_from / KT == t && (new_from % KT) / kPage == pg;
+            if (mixed && dma_wave) patch_page(cur);  // wave-uniform, once per workgroup at most
+        }
         tile_barrier();
         if (((t + 1) & (IDS_BLOCK - 1)) == 0 && t + 1 < t_end) {
             if (paged && dma_wave) {
@@ -427,12 +548,12 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
         // one box).
         constexpr bool late_v = D == 256;
         if (late_v) {
-            if (dma_wave) issue_page(t + 1, ids0, nxt, 0);
+            if (dma_wave) issue_page(any, t + 1, ids0, nxt, 0);
         } else {
-            issue_tile(t + 1, ids0, ids1, nxt);
+            issue_tile(any, t + 1, ids0, ids1, nxt);
         }
         auto issue_v = [&]() {
-            if (late_v && dma_wave) issue_page(t + 1, ids1, nxt, 1);
+            if (late_v && dma_wave) issue_page(any, t + 1, ids1, nxt, 1);
         };
         const int tok0 = t * KT + KH * kh;
         if (tok0 < wave_end)
@@ -440,9 +561,20 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
         else
             issue_v();
     };
-    for (int t = t_begin; t < t_end; t += 2) {
-        step(t, buf0, buf1);
-        step(t + 1, buf1, buf0);
+    int t = t_begin;
+    if constexpr (kNew) {
+        // the steps that neither hold nor request a row of the chunk, in a loop
+        // without the selects between its rows and the pages (512 of
+        // 4096, 16 waves: 58.7 -> 55.9 us)
+        const int t_new = new_from / KT;
+        for (; t + 2 < t_new && t < t_end; t += 2) {
+            step(std::false_type{}, t, buf0, buf1);
+            step(std::false_type{}, t + 1, buf1, buf0);
+        }
+    }
+    for (; t < t_end; t += 2) {
+        step(std::bool_constant<kNew>{}, t, buf0, buf1);
+        step(std::bool_constant<kNew>{}, t + 1, buf1, buf0);
     }
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // the trailing (empty) loads have landed: LDS is free
 
@@ -463,7 +595,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
             for (int i = 0; i < 4; ++i) tsum += acc[db][i];
         if (__any(!(fabsf(tsum) <= __FLT_MAX__))) {
             float res[DB * 4 + 2];
-            prefill_exact_part<D, F16, KT>(p, qrow, head_off, s_row, kh, wave_end, t_begin, t_end, res);
+            prefill_exact_part<D, F16, KT>(p, qrow, head_off, hkv, s_row, kh, wave_end, t_begin, t_end, res);
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -507,6 +639,8 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     }
     if (kh == 1) hand_over(qblk);
     __syncthreads();
+    if constexpr (kNew)
+        if (kh != 0) append_chunk<D>(tid - 256, (KQ - 1) * 256);
     if (kh != 0 || !wave_has_rows) return;
     const lds_float* const xch = slot(qblk);
     const float m1 = lds_ml[qblk][0][lane], l1 = lds_ml[qblk][1][lane];
@@ -557,9 +691,9 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
 // (4 waves per SIMD: at config 4 36.2 us, against 41.9 us for the earlier
 // form of one 128 KB, 196-VGPR workgroup per CU running two query tiles of
 // 2 x 32 queries, A/B on one box); D = 256: 128 KB, one workgroup per CU.
-template <bool F16, bool kSplit>
-__global__ __launch_bounds__(512, 2) void paged_prefill_d128_kernel(AttnParams p, PrefillGrid gr) {
-    prefill_tiles<128, F16, kSplit, 2>(p, gr);
+template <bool F16, bool kSplit, bool kNew>
+__global__ __launch_bounds__(512, kNew ? 4 : 2) void paged_prefill_d128_kernel(AttnParams p, PrefillGrid gr, AppendArg<kNew>) {
+    prefill_tiles<128, F16, kSplit, 2, kNew>(p, gr);
 }
 // 16 waves on 128-key tiles, one workgroup per CU: the same waves per CU as
 // two workgroups of the kernel above, for launches that have only one for
@@ -571,13 +705,13 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_d128_kernel(AttnParams p
 // tiles save (16 q / 8 kv heads, 1024 of 1024: 16.0 against 15.7 us, 100 of 1100
 // 16.0 against 15.6, 600 of 1500 18.9 against 19.7; 40 of 40: 8.7 against 6.3).
 constexpr int kWideFrom = 1280;
-template <bool F16>
-__global__ __launch_bounds__(1024) void paged_prefill_d128_wide_kernel(AttnParams p, PrefillGrid gr) {
-    prefill_tiles<128, F16, false, 4>(p, gr);
+template <bool F16, bool kNew>
+__global__ __launch_bounds__(1024) void paged_prefill_d128_wide_kernel(AttnParams p, PrefillGrid gr, AppendArg<kNew>) {
+    prefill_tiles<128, F16, false, 4, kNew>(p, gr);
 }
-template <bool F16, bool kSplit>
-__global__ __launch_bounds__(512) void paged_prefill_d256_kernel(AttnParams p, PrefillGrid gr) {
-    prefill_tiles<256, F16, kSplit, 2>(p, gr);
+template <bool F16, bool kSplit, bool kNew>
+__global__ __launch_bounds__(512) void paged_prefill_d256_kernel(AttnParams p, PrefillGrid gr, AppendArg<kNew>) {
+    prefill_tiles<256, F16, kSplit, 2, kNew>(p, gr);
 }
 
 // Merge of the key splits: 4 dims per lane (D / 4 lanes per row), kMergeU
@@ -632,23 +766,28 @@ __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(Attn
                                                  pack2(Elem<F16>::out(O[2] * inv), Elem<F16>::out(O[3] * inv)));
 }
 
-template <int D, bool F16>
-int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, hipStream_t stream) {
+bool wide_launch(const AttnParams& p, const PrefillGrid& gr, int head_dim) {
+    return head_dim == 128 && gr.n_splits == 1 && p.n_cached >= kWideFrom &&
+           int64_t(gr.n_rt) * gr.batch * p.Hkv <= device_cu_count();
+}
+
+template <int D, bool F16, bool kNew>
+int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, const AppendArg<kNew>& pa, hipStream_t stream) {
     const int64_t rows = int64_t(p.S) * p.G, units = int64_t(gr.batch) * p.Hkv;
     const int64_t wgs = gr.n_rt * units * gr.n_splits;
     const bool split = gr.n_splits > 1;
-    void (*k)(AttnParams, PrefillGrid);
+    void (*k)(AttnParams, PrefillGrid, AppendArg<kNew>);
     int threads = 512;
     if constexpr (D == 128) {
-        k = split ? paged_prefill_d128_kernel<F16, true> : paged_prefill_d128_kernel<F16, false>;
-        if (!split && wgs <= device_cu_count() && p.n_cached >= kWideFrom) {
-            k = paged_prefill_d128_wide_kernel<F16>;
+        k = split ? paged_prefill_d128_kernel<F16, true, kNew> : paged_prefill_d128_kernel<F16, false, kNew>;
+        if (wide_launch(p, gr, D)) {
+            k = paged_prefill_d128_wide_kernel<F16, kNew>;
             threads = 1024;
         }
     } else {
-        k = split ? paged_prefill_d256_kernel<F16, true> : paged_prefill_d256_kernel<F16, false>;
+        k = split ? paged_prefill_d256_kernel<F16, true, kNew> : paged_prefill_d256_kernel<F16, false, kNew>;
     }
-    hipLaunchKernelGGL(k, dim3(unsigned(wgs)), dim3(threads), 0, stream, p, gr);
+    hipLaunchKernelGGL(k, dim3(unsigned(wgs)), dim3(threads), 0, stream, p, gr, pa);
     GENLLM_LAUNCH_CHECK("paged_prefill kernel");
     if (!split) return GENLLM_OK;
     constexpr int kMergeWgRows = kMergeThreads / (D / 4);
@@ -656,6 +795,54 @@ int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, hipStream_t str
                        dim3(kMergeThreads), 0, stream, p, gr);
     GENLLM_LAUNCH_CHECK("paged_prefill_merge_kernel");
     return GENLLM_OK;
+}
+
+// The append runs inside the attention launch in the 16-wave form and where a
+// workgroup walks few key tiles: it saves a launch of 3.3-7 us, and costs a
+// step of the 8-wave forms about a tenth (the choice between the pages and the
+// chunk's rows).  Both kernels against the one, us (q / kv heads, head_dim,
+// queries of keys, key tiles of a workgroup): 32/8, 128, 512 of 4096 (16 waves)
+// 61.2, 55.9; 16/8, 128, 200 of 200 (4) 11.8, 9.1; 32/8, 128, 256 of 4096 (16)
+// 37.4, 36.1; 32/8, 128, 512 of 8192 (64) 93.1, 93.5; 32/8, 128, 1024 of 8192
+// (128) 154.1, 168.6; 8/2, 256, 128 of 1128 (3) 22.2, 20.6; 8/2, 256, 2048 of
+// 2048 (32) 54.6, 61.1.
+constexpr int kAppendTiles = 20;
+bool append_in_launch(const AttnParams& p, const PrefillGrid& gr, int head_dim) {
+    if (int64_t(2) * p.S * p.Hkv * (head_dim / 8) > INT32_MAX) return false;  // the copy counts in 32 bits
+    // an output that overlaps the chunk's rows must not be written before they are read
+    const auto overlaps = [&](const uint16_t* x) {
+        const uintptr_t o = reinterpret_cast<uintptr_t>(p.out), a = reinterpret_cast<uintptr_t>(x);
+        return o < a + size_t(p.S) * p.Hkv * head_dim * 2 && a < o + size_t(gr.batch) * p.S * p.Hq * head_dim * 2;
+    };
+    if (overlaps(p.k_new) || overlaps(p.v_new)) return false;
+    return wide_launch(p, gr, head_dim) || p.n_cached <= kAppendTiles * 64 * gr.n_splits;
+}
+
+int append_before(const AttnParams& p, const PrefillAppend& append, int head_dim, hipStream_t stream) {
+    AppendParams ap;
+    ap.upd = append.upd;
+    ap.k = p.k_new;
+    ap.v = p.v_new;
+    ap.k_tok_stride = ap.v_tok_stride = p.new_tok_stride;
+    ap.k_head_stride = ap.v_head_stride = p.new_head_stride;
+    ap.S = p.S;
+    ap.Hkv = p.Hkv;
+    ap.pos0 = p.new_from;
+    ap.nkv_tasks = (p.Hkv + 7) / 8;
+    ap.k_pool = p.k_pool_w;
+    ap.v_pool = p.v_pool_w;
+    ap.page_elems = p.page_elems;
+    ap.k_ids = p.k_ids_w;
+    ap.v_ids = p.v_ids_w;
+    ap.max_blocks = append.max_blocks;
+    return launch_kv_append(ap, head_dim, stream);
+}
+
+template <bool kNew>
+int launch_prefill(const AttnParams& p, const PrefillGrid& gr, const AppendArg<kNew>& pa, int head_dim, hipStream_t stream) {
+    if (head_dim == 128)
+        return p.f16 ? launch_prefill_d<128, true, kNew>(p, gr, pa, stream) : launch_prefill_d<128, false, kNew>(p, gr, pa, stream);
+    return p.f16 ? launch_prefill_d<256, true, kNew>(p, gr, pa, stream) : launch_prefill_d<256, false, kNew>(p, gr, pa, stream);
 }
 
 int resident_workgroups(int head_dim) { return device_cu_count() * (head_dim == 128 ? 2 : 1); }
@@ -709,7 +896,7 @@ int prefill_splits(int64_t units, int64_t rows, int n_cached, int head_dim, size
 }
 
 int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream, const PrefillBatch& b, float* ws,
-                         size_t ws_bytes) {
+                         size_t ws_bytes, const PrefillAppend* append) {
     if (head_dim != 128 && head_dim != 256) return fail(GENLLM_ERR_UNSUPPORTED, "paged prefill: head_dim must be 128 or 256");
     if (p.S <= 0 || p.n_pages <= 0 || b.n <= 0) return GENLLM_OK;
     const int64_t rows = int64_t(p.S) * p.G;
@@ -741,8 +928,17 @@ int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream, 
         gr.by_units = FastDiv(uint32_t(gr.batch * p.Hkv));
         gr.by_hkv = FastDiv(uint32_t(p.Hkv));
         gr.by_splits = FastDiv(uint32_t(gr.n_splits));
-        const int rc = head_dim == 128 ? (p.f16 ? launch_prefill_d<128, true>(pb, gr, stream) : launch_prefill_d<128, false>(pb, gr, stream))
-                                       : (p.f16 ? launch_prefill_d<256, true>(pb, gr, stream) : launch_prefill_d<256, false>(pb, gr, stream));
+        // The first launch appends, where that pays (append_in_launch); the rows
+        // are in their pages before a further one.
+        int rc = GENLLM_OK;
+        if (append && b0 == 0 && append_in_launch(pb, gr, head_dim)) {
+            rc = launch_prefill<true>(pb, gr, *append, head_dim, stream);
+        } else {
+            if (append && b0 == 0) rc = append_before(p, *append, head_dim, stream);
+            pb.k_new = pb.v_new = nullptr;
+            pb.new_from = INT32_MAX;
+            if (rc == GENLLM_OK) rc = launch_prefill<false>(pb, gr, NoAppend{}, head_dim, stream);
+        }
         if (rc) return rc;
     }
     return GENLLM_OK;

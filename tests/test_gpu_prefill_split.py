@@ -123,3 +123,41 @@ def test_small_row_tiles_vs_oracle(orc, Hq, Hkv, D, S, N, causal):
     q = synth.normal_bf16(8300 + N, (Hq, S, D))
     assert_attn_close(run_prefill(ctx, q, causal), ctx.oracle(q, causal), f"row tiles Hq{Hq} Hkv{Hkv} D{D} S{S} N{N}")
     ctx.close()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,S,prefix,f16,over", [
+    (4, 2, 128, 9, 7, False, None),      # the chunk starts and ends inside the first page
+    (4, 2, 128, 33, 0, False, None),     # no earlier tokens
+    (4, 1, 256, 40, 75, False, None),    # head_dim 256, starts inside a page
+    (2, 2, 128, 1290, 24, False, None),  # 16-wave form, nearly every tile the chunk's own
+    (2, 2, 128, 50, 1281, True, None),   # split, fp16: the last split holds the chunk
+    (2, 1, 128, 16, 64, False, None),    # whole pages
+    (1, 1, 128, 4120, 3, False, None),   # more pages than the launch arguments hold
+    (8, 2, 256, 30, 1500, False, None),
+    (2, 2, 128, 60, 100, False, "k"),    # the output over the chunk's K rows: appended before
+    (2, 2, 128, 60, 100, False, "v"),
+])
+def test_chunk_append_and_attention(orc, Hq, Hkv, D, S, prefix, f16, over):
+    """A chunk's rows reach their page slots and the table bit for bit, and the
+    attention sees them, whether one launch does both or two."""
+    N = prefix + S
+    mgr, ref = make(orc, Hkv, D, (N + 15) // 16 + 1, 600 + N, orc.F16 if f16 else orc.BF16)
+    gen = synth.normal_f16 if f16 else synth.normal_bf16
+    dev = paged.to_device_f16 if f16 else paged.to_device_bf16
+    if prefix:
+        k, v = gen(610 + N, (Hkv, prefix, D)), gen(611 + N, (Hkv, prefix, D))
+        mgr.append_kv_from_pos(0, dev(k), dev(v), 0)
+        ref.append_kv_from_pos(0, k, v, 0)
+    q, k, v = (gen(620 + N + i, (1, h, S, D)) for i, h in enumerate((Hq, Hkv, Hkv)))
+    qd, kd, vd = dev(q), dev(k), dev(v)
+    out = {None: torch.zeros_like(qd), "k": kd, "v": vd}[over]
+    paged.paged_attention(mgr, 0, qd, kd, vd, out, Hq // Hkv, scale_for(D))
+    torch.cuda.synchronize()
+    want, rc = ref.paged_attention(0, q, k, v, Hq // Hkv, scale_for(D), True, dtype=orc.F16 if f16 else orc.BF16)
+    assert rc == 0
+    (assert_attn_close_f16 if f16 else assert_attn_close)(paged.to_host_bits(out), want, f"chunk S{S} prefix {prefix} D{D}")
+    for which in (0, 1):
+        assert np.array_equal(mgr.read_pool(0, which), ref.pool_array(0, which)), f"pool {which}"
+    for got, table in zip(mgr.read_device_table(0), ref.page_table(0)):
+        assert np.array_equal(got, table)
+    mgr.close()
