@@ -136,7 +136,7 @@ __device__ __forceinline__ void tile_barrier() {
 // O^T values of the lane's dims 16 db + 4 g + i, then m (log2 units) and l
 // (the row's, in lane g = 0; 0 elsewhere, as the hand-over adds the four
 // lanes).  Called only by waves whose tiled state came out NaN or infinite.
-template <int D, bool F16, int KT>
+template <int D, bool F16, int KT, bool kNew>
 __device__ __forceinline__ void prefill_exact_part(const AttnParams& p, const uint16_t* qrow, int64_t kv_off, int hkv, int s_row,
                                                    int kh, int wave_end, int t_begin, int t_end, float* res) {
     using E = Elem<F16>;
@@ -156,7 +156,7 @@ __device__ __forceinline__ void prefill_exact_part(const AttnParams& p, const ui
             if (tok >= wave_end) break;  // wave-uniform
             const int64_t in_page = int64_t(tok % kPage) * p.kv_row;
             const uint16_t *krow, *vrow;
-            if (tok >= p.new_from) {  // appended by this call: its pages may not be written yet
+            if (kNew && tok >= p.new_from) {  // appended by this call: its pages may not be written yet
                 const int64_t at = hkv * p.new_head_stride + int64_t(tok - p.new_from) * p.new_tok_stride;
                 krow = p.k_new + at;
                 vrow = p.v_new + at;
@@ -390,29 +390,36 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     // kAny: the page may hold tokens of the chunk.
     auto issue_page = [&](auto any, int t, int ids, lds_char* buf, int kindx) {  // K (0) or V (1) rows of page pg of tile t
         constexpr bool kAny = decltype(any)::value;
-        const uint16_t* src = (kindx ? p.v_pool : p.k_pool) + head_off;
         const int tok_page = t * KT + kPage * pg;
-        int valid = min(max(kv_end - tok_page, 0), kPage);
-        int64_t base = paged ? int64_t(__builtin_amdgcn_readlane(ids, t & (IDS_BLOCK - 1))) * page_elems
-                             : int64_t(tok_page) * kv_row;
-        int row_bytes = kv_row_bytes, less = 0;
-        if constexpr (kAny) {
+        if constexpr (!kAny) {
+            const uint16_t* const src = (kindx ? p.v_pool : p.k_pool) + head_off;
+            const int valid = min(max(kv_end - tok_page, 0), kPage);
+            const uint32_t span = uint32_t(__builtin_amdgcn_readfirstlane(valid > 0 ? (valid - 1) * kv_row_bytes + ROWB : 0));
+            const int64_t base = paged ? int64_t(__builtin_amdgcn_readlane(ids, t & (IDS_BLOCK - 1))) * page_elems
+                                       : int64_t(tok_page) * kv_row;
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(src + base), 0, span, kBufferFlags);
+#pragma unroll
+            for (int e = 0; e < NI; ++e)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    r, (__attribute__((address_space(3))) void*)(buf + (kindx * TILEB + pg * (kPage * ROWB) + e * 1024)), 16,
+                    dma_off[e], 0, 0, 0);
+        } else {
             const int ahead = tok_page - new_from;
             const bool fresh = ahead >= 0;
-            src = fresh ? (kindx ? v_chunk : k_chunk) : src;
-            base = fresh ? int64_t(tok_page) * D : base;
-            row_bytes = fresh ? ROWB : kv_row_bytes;
-            valid = fresh ? valid : min(valid, -ahead);
-            less = kv_row_bytes - row_bytes;
-        }
-        const uint32_t span = uint32_t(__builtin_amdgcn_readfirstlane(valid > 0 ? (valid - 1) * row_bytes + ROWB : 0));
-        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(src + base), 0, span, kBufferFlags);
-        const uint32_t lane_less = kAny ? uint32_t(lane / LPR) * uint32_t(less) : 0;
+            const uint16_t* const src = fresh ? (kindx ? v_chunk : k_chunk) : (kindx ? p.v_pool : p.k_pool) + head_off;
+            const int64_t base = fresh ? int64_t(tok_page) * D
+                                       : int64_t(__builtin_amdgcn_readlane(ids, t & (IDS_BLOCK - 1))) * page_elems;
+            const int row_bytes = fresh ? ROWB : kv_row_bytes, less = kv_row_bytes - row_bytes;
+            const int rows = min(max(kv_end - tok_page, 0), kPage), valid = fresh ? rows : min(rows, -ahead);
+            const uint32_t span = uint32_t(__builtin_amdgcn_readfirstlane(valid > 0 ? (valid - 1) * row_bytes + ROWB : 0));
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(src + base), 0, span, kBufferFlags);
+            const uint32_t lane_less = uint32_t(lane / LPR) * uint32_t(less);
 #pragma unroll
-        for (int e = 0; e < NI; ++e)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                r, (__attribute__((address_space(3))) void*)(buf + (kindx * TILEB + pg * (kPage * ROWB) + e * 1024)), 16,
-                kAny ? dma_off[e] - lane_less - uint32_t(RPI * e) * uint32_t(less) : dma_off[e], 0, 0, 0);
+            for (int e = 0; e < NI; ++e)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    r, (__attribute__((address_space(3))) void*)(buf + (kindx * TILEB + pg * (kPage * ROWB) + e * 1024)), 16,
+                    dma_off[e] - lane_less - uint32_t(RPI * e) * uint32_t(less), 0, 0, 0);
+        }
     };
     // The chunk's rows of the page where it starts inside a page, into the
     // landed tile (the loads above left zeros there).
@@ -595,7 +602,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
             for (int i = 0; i < 4; ++i) tsum += acc[db][i];
         if (__any(!(fabsf(tsum) <= __FLT_MAX__))) {
             float res[DB * 4 + 2];
-            prefill_exact_part<D, F16, KT>(p, qrow, head_off, hkv, s_row, kh, wave_end, t_begin, t_end, res);
+            prefill_exact_part<D, F16, KT, kNew>(p, qrow, head_off, hkv, s_row, kh, wave_end, t_begin, t_end, res);
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
