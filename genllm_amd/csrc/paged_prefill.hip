@@ -812,8 +812,10 @@ int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, const AppendArg
 // 61.2, 55.9; 16/8, 128, 200 of 200 (4) 11.8, 9.1; 32/8, 128, 256 of 4096 (16)
 // 37.4, 36.1; 32/8, 128, 512 of 8192 (64) 93.1, 93.5; 32/8, 128, 1024 of 8192
 // (128) 154.1, 168.6; 8/2, 256, 128 of 1128 (3) 22.2, 20.6; 8/2, 256, 2048 of
-// 2048 (32) 54.6, 61.1.
-constexpr int kAppendTiles = 20;
+// 2048 (32) 54.6, 61.1.  Unsplit and with the keys still in the caches the line
+// lies lower (32/8, 128, chunks of 269 of 536..1326: 82.5 us a session with
+// kAppendTiles 8, 85.9 with 20).
+constexpr int kAppendTiles = 8, kAppendSplitTiles = 20;
 bool append_in_launch(const AttnParams& p, const PrefillGrid& gr, int head_dim) {
     if (int64_t(2) * p.S * p.Hkv * (head_dim / 8) > INT32_MAX) return false;  // the copy counts in 32 bits
     // an output that overlaps the chunk's rows must not be written before they are read
@@ -822,7 +824,8 @@ bool append_in_launch(const AttnParams& p, const PrefillGrid& gr, int head_dim) 
         return o < a + size_t(p.S) * p.Hkv * head_dim * 2 && a < o + size_t(gr.batch) * p.S * p.Hq * head_dim * 2;
     };
     if (overlaps(p.k_new) || overlaps(p.v_new)) return false;
-    return wide_launch(p, gr, head_dim) || p.n_cached <= kAppendTiles * 64 * gr.n_splits;
+    return wide_launch(p, gr, head_dim) ||
+           p.n_cached <= int64_t(gr.n_splits > 1 ? kAppendSplitTiles : kAppendTiles) * 64 * gr.n_splits;
 }
 
 int append_before(const AttnParams& p, const PrefillAppend& append, int head_dim, hipStream_t stream) {
@@ -887,11 +890,12 @@ int prefill_splits(int64_t units, int64_t rows, int n_cached, int head_dim, size
     const bool d128 = head_dim == 128;
     const double kTileUs = d128 ? 0.8 : 1.45, kSplitTileUs = d128 ? 0.85 : 1.45, kPairTileUs = 1.25;
     const double kMergeUs = 6.0, kMergeUsPerMB = 0.46;
+    const double kUnsplit = 0.85;  // less where the keys are still in the caches
     const int64_t cus = device_cu_count(), wgs = (rows + QT - 1) / QT * units;
     const int64_t tiles = (int64_t(n_cached) + 63) / 64;
     const int64_t most = std::min<int64_t>({resident_workgroups(head_dim) / wgs, tiles, kMaxPrefillSplits});
     int best = 1;
-    double best_us = double(tiles) * kTileUs;
+    double best_us = kUnsplit * double(tiles) * kTileUs;
     for (int64_t ns = 2; ns <= most; ++ns) {
         const double bytes = double(ns * units * rows) * (head_dim + 2) * sizeof(float);
         if (bytes > double(ws_bytes)) break;
