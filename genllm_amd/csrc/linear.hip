@@ -21,7 +21,7 @@
 // forms of the 8-element group agree.)
 //
 // More rows: rocBLAS gemm_ex, bf16 inputs and fp32 compute.  With a bias, the
-// fp32 result goes to the caller's workspace and linear_epilogue_kernel adds
+// fp32 result goes to the caller's workspace and an epilogue kernel adds
 // the bias in fp32 and rounds once; without one (Qwen3's projections), rocBLAS
 // writes bf16 directly, rounding the fp32 result once to nearest even (an
 // fp32 subnormal result stays a bf16 subnormal where the reference flushes it
@@ -363,6 +363,32 @@ __global__ __launch_bounds__(256) void linear_epilogue_kernel(const float* __res
     }
 }
 
+// The same where 4 columns make an aligned load: thread -> 4 columns of
+// kEpiRows rows, so the bias is read once and no index needs a division.
+// Bound by memory (6 bytes per element): 1500 x 4096 8.7 us, 1500 x 1024 2.7 us
+// (kernel trace); 11.4 and 3.4 us in the kernel above, which stays for the
+// widths and pointers that do not allow it.
+constexpr int kEpiRows = 4;
+__global__ __launch_bounds__(256) void linear_epilogue4_kernel(const float* __restrict__ acc,
+                                                               const uint16_t* __restrict__ bias,
+                                                               uint16_t* __restrict__ out, int64_t rows, int cols) {
+    const int c = 4 * int(blockIdx.x * 256 + threadIdx.x);
+    if (c >= cols) return;
+    const uint2 b = *reinterpret_cast<const uint2*>(bias + c);
+    const float bv[4] = {bf16_lo(b.x), bf16_hi(b.x), bf16_lo(b.y), bf16_hi(b.y)};
+    for (int64_t r0 = int64_t(blockIdx.y) * kEpiRows; r0 < rows; r0 += int64_t(gridDim.y) * kEpiRows) {
+        f32x4_t v[kEpiRows];
+#pragma unroll
+        for (int u = 0; u < kEpiRows; ++u)
+            if (r0 + u < rows) v[u] = *reinterpret_cast<const f32x4_t*>(acc + (r0 + u) * cols + c);
+#pragma unroll
+        for (int u = 0; u < kEpiRows; ++u)
+            if (r0 + u < rows)
+                *reinterpret_cast<uint2*>(out + (r0 + u) * cols + c) =
+                    make_uint2(bf16_pair_out(v[u][0] + bv[0], v[u][1] + bv[1]), bf16_pair_out(v[u][2] + bv[2], v[u][3] + bv[3]));
+    }
+}
+
 // one rocBLAS handle per device, created on first use
 std::mutex g_blas_mu;
 std::map<int, rocblas_handle> g_blas;
@@ -456,6 +482,13 @@ int launch_linear(const uint16_t* x, const uint16_t* w, const uint16_t* bias, ui
         rocblas_int(cols), rocblas_datatype_f32_r, rocblas_gemm_algo_standard, 0, 0);
     if (st != rocblas_status_success)
         return fail(GENLLM_ERR_HIP, std::string("linear: rocblas_gemm_ex failed: ") + rocblas_status_to_string(st));
+    const auto aligned = [](const void* x, uintptr_t a) { return (reinterpret_cast<uintptr_t>(x) & (a - 1)) == 0; };
+    if (cols % 4 == 0 && cols <= INT32_MAX - 1024 && aligned(acc, 16) && aligned(bias, 8) && aligned(out, 8)) {
+        const dim3 grid(unsigned((cols / 4 + 255) / 256), unsigned(std::min<int64_t>((rows + kEpiRows - 1) / kEpiRows, 16384)));
+        hipLaunchKernelGGL(linear_epilogue4_kernel, grid, dim3(256), 0, stream, acc, bias, out, rows, int(cols));
+        GENLLM_LAUNCH_CHECK("linear_epilogue4_kernel");
+        return GENLLM_OK;
+    }
     const int64_t n = rows * cols;
     const unsigned grid = unsigned(std::min<int64_t>((n + 255) / 256, 4096));
     hipLaunchKernelGGL(linear_epilogue_kernel, dim3(grid), dim3(256), 0, stream, acc, bias, out, n, int(cols));
