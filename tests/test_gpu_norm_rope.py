@@ -56,3 +56,38 @@ def test_apply_rope_widths(orc, H, S, D, rope_dim, offset):
     want = orc.apply_rope_partial(x, cos, sin, 3)
     assert np.array_equal(paged.to_host_bits(out), want)
     assert np.array_equal(paged.to_host_bits(xd), want)
+
+
+def same_but_nan(got, want):
+    """Bit-equal, NaNs in the same places (their sign and payload are not fixed)."""
+    g, w = synth.bf16_bits_to_f32(got), synth.bf16_bits_to_f32(want)
+    return np.array_equal(np.isnan(g), np.isnan(w)) and np.array_equal(got[~np.isnan(w)], want[~np.isnan(w)])
+
+
+SPECIALS = np.array([0x7FC0, 0xFF81, 0x7F80, 0xFF80, 0x0001, 0x8001, 0x007F, 0x0080, 0x7F7F, 0xFF7F, 0x8000], dtype=np.uint16)
+
+
+def with_specials(seed, shape):
+    x = synth.normal_bf16(seed, shape).reshape(-1)
+    r = np.random.default_rng(seed)
+    at = r.choice(x.size, 200, replace=False)
+    x[at] = r.choice(SPECIALS, 200)
+    return x.reshape(shape)
+
+
+@pytest.mark.parametrize("hidden,rows", [(128, 500), (2560, 300), (520, 300)])
+def test_rms_norm_special_values(orc, hidden, rows):
+    x = with_specials(hidden, (rows, hidden))
+    w = synth.uniform_f32(hidden + 1, (hidden,), 0.5, 1.5)
+    out = torch.empty((rows, hidden), dtype=torch.bfloat16, device="cuda")
+    paged.rms_norm(out, paged.to_device_bf16(x), torch.from_numpy(w).cuda(), 1e-6)
+    assert same_but_nan(paged.to_host_bits(out), orc.rms_norm(x, w, 1e-6))
+
+
+@pytest.mark.parametrize("H,S,D,rope_dim", [(5, 900, 128, 128), (3, 900, 256, 64)])
+def test_apply_rope_special_values(orc, H, S, D, rope_dim):
+    x = with_specials(H * S, (H, S, D))
+    cos, sin = paged.rope_cache(1e6, rope_dim, S)
+    out = torch.empty((H, S, D), dtype=torch.bfloat16, device="cuda")
+    paged.apply_rope(out, paged.to_device_bf16(x), torch.from_numpy(cos).cuda(), torch.from_numpy(sin).cuda(), 0)
+    assert same_but_nan(paged.to_host_bits(out), orc.apply_rope_partial(x, cos, sin, 0))
