@@ -93,10 +93,11 @@ struct AttnParams {
     // nothing; otherwise the merge kernel advances pos by S (without one, the
     // last split workgroup to finish does).
     int32_t* step = nullptr;
-    // fused append (decode of the op): tokens at positions >= new_from are read
-    // from k_new / v_new ([Hkv][S][D], strides in elements) instead of the
-    // pools and written into the pools by the wave that reads their page; page
-    // ids opened by this call come in `upd` and are written to the tables.
+    // fused append (the op): tokens at positions >= new_from are read from
+    // k_new / v_new ([Hkv][S][D], strides in elements) instead of the pools and
+    // written into the pools, in the decode kernel by the wave that reads their
+    // page; page ids opened by this call come in `upd` (prefill: PrefillAppend)
+    // and are written to the tables.
     const uint16_t* k_new = nullptr;
     const uint16_t* v_new = nullptr;
     int64_t new_head_stride = 0, new_tok_stride = 0;

@@ -62,9 +62,11 @@ int genllm_kv_init_layer(genllm_kv *kv, int32_t layer, int32_t n_kv_heads, int32
  * K pool and the V pool (max_blocks pages each, 256-byte aligned) from the
  * kv_cache pool -- exactly the 2 * max_blocks * block_bytes per layer the
  * reference scheduler sizes it for (scheduler.cpp:62-79, 371).  The device
- * page table (max_blocks entries), its pinned host staging and the manager's
- * decode workspace are allocated separately, here, once: the op itself never
- * allocates, frees or synchronises. */
+ * page table (max_blocks entries), its pinned host staging, the manager's
+ * decode workspace and, for more than 256 tokens, the layer's scratch for
+ * prefill chunks whose keys are split over workgroups (17 MB; without memory
+ * for it the chunks run unsplit) are allocated separately, here, once: the op
+ * itself never allocates, frees or synchronises. */
 int genllm_kv_reserve_layer(genllm_kv *kv, int32_t layer, int32_t max_blocks);
 /* PagedAttentionManager::is_active, page_attention.h:82-85; *active = 0/1 */
 int genllm_kv_is_active(genllm_kv *kv, int32_t layer, int32_t *active);
@@ -136,7 +138,10 @@ int genllm_kv_block_free(genllm_kv *kv, int32_t layer, int32_t which, int32_t id
  * and 256 (Qwen3.5, Qwen35.hpp:14-16) are served; any other returns
  * GENLLM_ERR_UNSUPPORTED (the CUDA op throws for head_dim != 128,
  * attention.cu:511).  Chunks of up to 16 (query, q-head) rows per kv head run
- * the split-K decode kernel, longer chunks the MFMA prefill kernel.  Every
+ * the split-K decode kernel, longer chunks the MFMA prefill kernels, with the
+ * keys split over workgroups where the chunk alone would leave the GPU idle.
+ * k and v are read while out is written in the decode kernel's range; longer
+ * chunks take an out that overlaps them as well.  Every
  * argument check and the split plan run before the layer changes: a call that
  * returns an error leaves num_cached, the page tables and the block pools as
  * they were. */
@@ -260,7 +265,8 @@ int genllm_paged_decode(const void *q, int64_t q_head_stride, int64_t q_tok_stri
 /* No counterpart in the reference: a tuning and test hook for the decode
  * kernels of this library (genllm_paged_decode, _noalloc, the op and its
  * device-position steps), process-wide, for later calls.  pages_per_split > 0
- * forces the split size (0: automatic, about one workgroup per CU).  merge:
+ * forces the split size (0: automatic, about one workgroup per CU, one split
+ * for a few pages).  merge:
  * 0 = a merge kernel after the split kernel (default), 1 = the last split
  * workgroup of each kv head to finish merges it in the same launch.
  * heads_per_workgroup: kv heads one split workgroup reads; 0 = automatic (4
