@@ -5,10 +5,10 @@
 // at q_abs = n_cached - S + s and attends keys 0..q_abs (causal, :164-181),
 // kv head = q head / groups (:158).
 //
-// Rows: the S x groups (query, q head) pairs of a kv head, q heads fastest, in
-// row tiles of 64 (fewer where CUs would stay idle), so a short chunk fills its tiles and the q heads of a kv
-// head share their key tiles.  Grid: row tiles x (batch entry, kv head) pairs,
-// workgroups of 8 waves: the long half of the row tiles from the last down,
+// Rows: the queries of a q head or, in short chunks and split launches, the S x
+// groups (query, q head) pairs of a kv head, q heads fastest, in row tiles of 64
+// (fewer where CUs would stay idle), so a short chunk fills its tiles.  Grid: row
+// tiles x (batch entry, head) pairs, workgroups of 8 waves: the long half of the row tiles from the last down,
 // then the short half from the first up; or, where that would leave the chip
 // idle, row tiles x key splits, merged by a second kernel (prefill_splits).
 // All batch entries go in one launch: two prompts of 1000 tokens (16 q / 8 kv
@@ -91,7 +91,10 @@ struct PrefillGrid {
     int64_t q_batch = 0, o_batch = 0, kv_batch = 0;
     int32_t batch = 1, n_splits = 1;
     int32_t tile_rows = QT;    // rows per row tile: 16, 32 or 64
-    FastDiv by_g, by_units, by_hkv, by_splits;  // groups, batch x kv heads, kv heads, n_splits
+    int32_t pack = 1;          // q heads whose rows share row tiles: the groups of a kv head, or 1
+    int32_t units = 1;         // batch entries x (q heads / pack)
+    // pack, units, q heads / pack, groups / pack, kv heads, n_splits
+    FastDiv by_pack, by_units, by_heads, by_groups, by_hkv, by_splits;
     int32_t n_rt = 0;                           // row tiles of a kv head
     float* partial = nullptr;  // n_splits > 1: o [split][unit][row][D], then {m, l} [split][unit][row]
 };
@@ -287,17 +290,21 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int qblk = wv & 3, kh = wv >> 2;  // row block, key part (waves w, w + 4, ... share a SIMD)
     const int n16 = lane & 15, g = lane >> 4;
-    const int G = p.G, R = p.S * G;  // rows of a kv head: row r is q head r % G of query r / G
+    const int pack = gr.pack, R = p.S * pack;  // rows of a unit: row r is q head r % pack of query r / pack
     const int tile_rows = gr.tile_rows;
     const int n_rt = gr.n_rt;
-    // Workgroup i runs on XCD i % 8: with the (batch entry, kv head) pairs
-    // fastest and 8 kv heads, XCD x holds kv head x and its tiles are read
-    // through one L2 (config 4: FETCH_SIZE 16.2 against 24.2 MiB per launch
+    // Workgroup i runs on XCD i % 8: with the (batch entry, head) pairs fastest
+    // and 8 kv heads, XCD x holds kv head x (single q heads, in multiples of 8:
+    // q heads [x heads / 8, (x + 1) heads / 8)) and its tiles are read through
+    // one L2 (config 4: FETCH_SIZE 16.2 against 24.2 MiB per launch
     // with a kv head's rows spread over two XCDs)
-    const int units = gr.batch * p.Hkv;
+    const int units = gr.units, heads = kSplit ? p.Hkv : pack == 1 ? p.Hq : p.Hkv;
     const int rank = gr.by_units(int(blockIdx.x));
     const int unit = int(blockIdx.x) - rank * units;
-    const int bat = gr.by_hkv(unit), hkv = unit - bat * p.Hkv;
+    const int bat = gr.by_heads(unit);
+    int hg = unit - bat * heads;  // the unit's heads: hg * pack .. + pack - 1
+    if (!kSplit && pack == 1 && (heads & 7) == 0) hg = (hg & 7) * (heads >> 3) + (hg >> 3);
+    const int hkv = kSplit ? hg : gr.by_groups(hg);
     // Unsplit: the first half of the grid runs the row tiles with the most
     // keys, from the last tile down; the second half the others from the first
     // tile up, so that workgroups i and i + half the grid -- the two a CU holds
@@ -315,8 +322,8 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     // Q^T operands: lane -> row q0 + n16, dims 32ks + 8g..+7 (a row past the
     // last one loads the last row: its column stays finite and is not written)
     const int row = min(q0 + n16, R - 1);
-    const int s_row = gr.by_g(row);  // the row's query
-    const uint16_t* const qrow = p.q + bat * gr.q_batch + int64_t(hkv * G + (row - s_row * G)) * p.q_head_stride +
+    const int s_row = gr.by_pack(row);  // the row's query
+    const uint16_t* const qrow = p.q + bat * gr.q_batch + int64_t(hg * pack + (row - s_row * pack)) * p.q_head_stride +
                                  int64_t(s_row) * p.q_tok_stride;
     uint4 qb[KS];  // raw 16-bit elements
 #pragma unroll
@@ -329,7 +336,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
 #pragma unroll
     for (int db = 0; db < DB; ++db) acc[db] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int s_last = gr.by_g(min(rt * tile_rows + tile_rows, R) - 1);  // last query of the workgroup
+    const int s_last = gr.by_pack(min(rt * tile_rows + tile_rows, R) - 1);  // last query of the workgroup
     const int kv_last = p.causal ? min(qabs0 + s_last + 1, n_cached) : n_cached;
     const int n_tiles = (kv_last + KT - 1) / KT;
     // key tiles [t_begin, t_end) of this workgroup; keys at or past kv_end are
@@ -340,9 +347,9 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     const bool wave_has_rows = q0 < R && qblk * QW < tile_rows;
     // keys below wave_lim are visible to every row of the wave, keys at or
     // past wave_end to none of them (or not this split's)
-    const int wave_lim = p.causal ? min(qabs0 + gr.by_g(q0) + 1, n_cached) : n_cached;
+    const int wave_lim = p.causal ? min(qabs0 + gr.by_pack(q0) + 1, n_cached) : n_cached;
     const int wave_end = !wave_has_rows ? 0
-                         : p.causal     ? min(qabs0 + gr.by_g(min(q0 + QW, R) - 1) + 1, kv_end)
+                         : p.causal     ? min(qabs0 + gr.by_pack(min(q0 + QW, R) - 1) + 1, kv_end)
                                         : kv_end;
 
     // ---- staging: wave w < 4 moves page w of each tile, its K rows, then its
@@ -674,8 +681,8 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
         return;
     }
     const float inv = 1.0f / lt;
-    const int s_out = gr.by_g(r_out);
-    uint16_t* orow = p.out + bat * gr.o_batch + int64_t(hkv * G + (r_out - s_out * G)) * p.o_head_stride +
+    const int s_out = gr.by_pack(r_out);
+    uint16_t* orow = p.out + bat * gr.o_batch + int64_t(hg * pack + (r_out - s_out * pack)) * p.o_head_stride +
                      int64_t(s_out) * p.o_tok_stride;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
@@ -765,7 +772,7 @@ __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(Attn
         M = bm;
     }
     const float inv = 1.0f / L;
-    const int unit = at / R, r = at - unit * R, s = gr.by_g(r);
+    const int unit = at / R, r = at - unit * R, s = gr.by_pack(r);
     const int bat = gr.by_hkv(unit), hkv = unit - bat * p.Hkv;
     uint16_t* const orow = p.out + bat * gr.o_batch + int64_t(hkv * G + (r - s * G)) * p.o_head_stride +
                            int64_t(s) * p.o_tok_stride + d0;
@@ -775,12 +782,12 @@ __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(Attn
 
 bool wide_launch(const AttnParams& p, const PrefillGrid& gr, int head_dim) {
     return head_dim == 128 && gr.n_splits == 1 && p.n_cached >= kWideFrom &&
-           int64_t(gr.n_rt) * gr.batch * p.Hkv <= device_cu_count();
+           int64_t(gr.n_rt) * gr.units <= device_cu_count();
 }
 
 template <int D, bool F16, bool kNew>
 int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, const AppendArg<kNew>& pa, hipStream_t stream) {
-    const int64_t rows = int64_t(p.S) * p.G, units = int64_t(gr.batch) * p.Hkv;
+    const int64_t rows = int64_t(p.S) * gr.pack, units = gr.units;
     const int64_t wgs = gr.n_rt * units * gr.n_splits;
     const bool split = gr.n_splits > 1;
     void (*k)(AttnParams, PrefillGrid, AppendArg<kNew>);
@@ -911,8 +918,8 @@ int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream, 
     if (head_dim != 128 && head_dim != 256) return fail(GENLLM_ERR_UNSUPPORTED, "paged prefill: head_dim must be 128 or 256");
     if (p.S <= 0 || p.n_pages <= 0 || b.n <= 0) return GENLLM_OK;
     const int64_t rows = int64_t(p.S) * p.G;
-    // entries per launch: a grid of at most 2^22 workgroups (HIP takes up to 2^32 threads)
-    const int64_t per = std::max<int64_t>(1, (int64_t(1) << 22) / ((rows + QT - 1) / QT * p.Hkv));
+    // entries per launch: a grid of about 2^21 workgroups at most (HIP takes up to 2^32 threads)
+    const int64_t per = std::max<int64_t>(1, (int64_t(1) << 21) / ((rows + QT - 1) / QT * p.Hkv));
     for (int64_t b0 = 0; b0 < b.n; b0 += per) {
         AttnParams pb = p;
         pb.q += b0 * b.q_stride;
@@ -926,17 +933,25 @@ int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream, 
         gr.kv_batch = b.kv_stride;
         gr.partial = ws;
         gr.n_splits = ws ? prefill_splits(int64_t(gr.batch) * p.Hkv, rows, p.n_cached, head_dim, ws_bytes) : 1;
+        // A split launch packs the q heads of a kv head into its row tiles, as
+        // does any chunk whose single heads would leave a twentieth more tiles.
+        // Otherwise each q head has its own (D = 256, 16 / 4 heads, 814 tokens
+        // 23.0 against 24.1 us; D = 128, 32 / 8, 700 tokens 14.1 against 14.4).
+        const bool own = gr.n_splits == 1 && (int64_t(p.S) + QT - 1) / QT * p.G * 20 <= (rows + QT - 1) / QT * 21;
+        gr.pack = own ? 1 : p.G;
+        gr.units = gr.batch * (own ? p.Hq : p.Hkv);
+        const int64_t unit_rows = own ? p.S : rows;
         // Where CUs would stay idle, smaller row tiles spread the rows over more
         // of them, fewer row blocks each (tiles of 16, 32 and 64 rows, us: 16 q
         // / 8 kv heads, 100 of 700 11.4, 11.5, 11.8; 500 of 1030 15.1, 15.3,
         // 15.6; 64 of 4000 37.5, 38.1, 39.0).
-        if (gr.n_splits == 1) {
-            const int64_t cus = device_cu_count(), units = int64_t(gr.batch) * p.Hkv;
-            for (int r = QT / 2; r >= QW && (rows + r - 1) / r * units <= cus; r /= 2) gr.tile_rows = r;
-        }
-        gr.n_rt = int32_t((rows + gr.tile_rows - 1) / gr.tile_rows);
-        gr.by_g = FastDiv(uint32_t(p.G));
-        gr.by_units = FastDiv(uint32_t(gr.batch * p.Hkv));
+        if (gr.n_splits == 1)
+            for (int r = QT / 2; r >= QW && (unit_rows + r - 1) / r * gr.units <= device_cu_count(); r /= 2) gr.tile_rows = r;
+        gr.n_rt = int32_t((unit_rows + gr.tile_rows - 1) / gr.tile_rows);
+        gr.by_pack = FastDiv(uint32_t(gr.pack));
+        gr.by_units = FastDiv(uint32_t(gr.units));
+        gr.by_heads = FastDiv(uint32_t(own ? p.Hq : p.Hkv));
+        gr.by_groups = FastDiv(uint32_t(own ? p.G : 1));
         gr.by_hkv = FastDiv(uint32_t(p.Hkv));
         gr.by_splits = FastDiv(uint32_t(gr.n_splits));
         // The first launch appends, where that pays (append_in_launch); the rows
