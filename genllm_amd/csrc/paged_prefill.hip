@@ -8,9 +8,10 @@
 // Rows: the queries of a q head or, in short chunks and split launches, the S x
 // groups (query, q head) pairs of a kv head, q heads fastest, in row tiles of 64
 // (fewer where CUs would stay idle), so a short chunk fills its tiles.  Grid: row
-// tiles x (batch entry, head) pairs, workgroups of 8 waves: the long half of the row tiles from the last down,
-// then the short half from the first up; or, where that would leave the chip
-// idle, row tiles x key splits, merged by a second kernel (prefill_splits).
+// tiles x (batch entry, head) pairs, workgroups of 8 waves: the long half of the
+// row tiles from the last down, then the short half from the first up; or, where
+// that would leave the chip idle, row tiles x key splits, merged by a second
+// kernel (prefill_splits).
 // All batch entries go in one launch: two prompts of 1000 tokens (16 q / 8 kv
 // heads of 128) 16.9 us in one launch of 512 workgroups, 29.5 us in two.
 // Wave w = qb + 4 kh owns row block qb (16 rows) of the tile and key

@@ -86,7 +86,12 @@ def test_split_prefill_special_values(orc, D, S, N):
     mgr.close()
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(3, 4, 2, 70, 128), (5, 2, 1, 1, 256)])
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [
+    (3, 4, 2, 70, 128),   # the q heads of a kv head packed into row tiles
+    (5, 2, 1, 1, 256),
+    (2, 16, 4, 64, 128),  # a row tile for each q head, heads in multiples of 8
+    (2, 6, 2, 127, 256),  # row tiles of single q heads, 6 of them
+])
 def test_flash_batch_in_one_launch(orc, B, Hq, Hkv, S, D):
     """Every batch entry of the non-paged op reads its own q, k and v rows."""
     q, k, v = (synth.normal_bf16(7000 + i, (B, h, S, D)) for i, h in enumerate((Hq, Hkv, Hkv)))
