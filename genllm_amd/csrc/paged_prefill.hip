@@ -732,6 +732,9 @@ __global__ __launch_bounds__(512) void paged_prefill_d256_kernel(AttnParams p, P
 // Merge of the key splits: 4 dims per lane (D / 4 lanes per row), kMergeU
 // splits in flight, with the log-sum-exp rule
 //   M = max m_s, L = sum l_s 2^(m_s - M), O = sum o_s 2^(m_s - M), out = O / L.
+// A split without a maximum (m_s = -inf) has weight 0, which its l and o are
+// multiplied by all the same: they are zeros where the row sees no key of the
+// split, but NaN where every score is NaN, and that NaN is the row's result.
 constexpr int kMergeThreads = 256, kMergeU = 8;
 template <int D, bool F16>
 __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(AttnParams p, PrefillGrid gr) {
@@ -754,21 +757,24 @@ __global__ __launch_bounds__(kMergeThreads) void paged_prefill_merge_kernel(Attn
             const int64_t off = int64_t(in ? s0 + u : s0) * rows;
             ov[u] = *reinterpret_cast<const f32x4_t*>(po + off * D);
             mv[u] = ml[off];
-            if (!in) mv[u].x = -INFINITY;
+            if (!in) {  // the first of them again: weighs nothing
+                ov[u] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                mv[u] = make_float2(-INFINITY, 0.0f);
+            }
         }
         float bm = M;
 #pragma unroll
         for (int u = 0; u < kMergeU; ++u) bm = fmaxf(bm, mv[u].x);
-        const float a = M == -INFINITY ? 0.0f : exp2_fast(M - bm);
+        const float ref = bm == -INFINITY ? 0.0f : bm;
+        const float a = exp2_fast(M - ref);  // 0 while M = -inf
         L *= a;
         O *= a;
 #pragma unroll
         for (int u = 0; u < kMergeU; ++u) {
-            const bool on = mv[u].x != -INFINITY;  // a split that saw no key weighs nothing
-            const float w = on ? exp2_fast(mv[u].x - bm) : 0.0f;
-            L += on ? mv[u].y * w : 0.0f;
+            const float w = exp2_fast(mv[u].x - ref);
+            L += mv[u].y * w;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) O[i] += on ? ov[u][i] * w : 0.0f;
+            for (int i = 0; i < 4; ++i) O[i] += ov[u][i] * w;
         }
         M = bm;
     }

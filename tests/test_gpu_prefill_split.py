@@ -3,15 +3,15 @@ splits their keys over workgroups and a second kernel merges the splits.
 Against the oracle op, at the edges of that path: rows that do not fill a row
 tile of 64 (query, q head) pairs, key counts on and off the 64-key tile, more
 than 64 key tiles (page ids come 64 tiles at a time, and a split may start or
-end inside such a block), fp16, several batch entries, not causal, and NaN and
-infinite inputs in the chunk's own rows.  Tolerances as everywhere (max-abs <=
+end inside such a block), fp16, several batch entries, not causal, NaN and
+infinite inputs in the chunk's own rows, and splits whose keys are all NaN.  Tolerances as everywhere (max-abs <=
 2^-7 max|ref| and rel-L2 <= 1e-2 in bf16, 2^-8 and 4e-3 in fp16)."""
 import numpy as np
 import pytest
 import torch
 
 from genllm_amd import paged, synth
-from helpers import assert_attn_close, assert_attn_close_f16, f32, scale_for
+from helpers import assert_attn_close, assert_attn_close_f16, f16 as as_f16, f32, scale_for
 from test_gpu_decode import Context
 from test_gpu_f16_batch import make
 from test_gpu_prefill import run_prefill
@@ -35,12 +35,14 @@ def chunk(orc, mgr, ref, Hq, Hkv, S, D, seed, f16=False, batch=1, causal=True, p
     return paged.to_host_bits(out), want
 
 
-def cached(orc, Hkv, D, N, S, seed, f16):
+def cached(orc, Hkv, D, N, S, seed, f16, plant=None):
     """A layer holding N - S tokens, written without attending over them."""
     mgr, ref = make(orc, Hkv, D, (N + 15) // 16 + 3, seed, orc.F16 if f16 else orc.BF16)
     gen = synth.normal_f16 if f16 else synth.normal_bf16
     dev = paged.to_device_f16 if f16 else paged.to_device_bf16
-    k, v = gen(seed + 5, (Hkv, N - S, D)), gen(seed + 6, (Hkv, N - S, D))
+    k, v = gen(seed + 5, (Hkv, N - S, D)).copy(), gen(seed + 6, (Hkv, N - S, D))
+    if plant:
+        plant(k)
     mgr.append_kv_from_pos(0, dev(k), dev(v), 0)
     ref.append_kv_from_pos(0, k, v, 0)
     return mgr, ref
@@ -83,6 +85,42 @@ def test_split_prefill_special_values(orc, D, S, N):
     assert nf.any() and np.array_equal(nf, ~np.isfinite(f32(got)))
     assert np.array_equal(got[nf] & 0x7FFF, want[nf] & 0x7FFF)
     assert_attn_close(np.where(nf, 0, got).astype(np.uint16), np.where(nf, 0, want).astype(np.uint16), f"special D{D}")
+    mgr.close()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,S,N,f16,first,last", [
+    (32, 8, 128, 8, 1089, False, 1088, 1088),   # 18 splits of a tile: the last one holds key 1088 alone
+    (8, 2, 256, 8, 1089, False, 1088, 1088),
+    (32, 8, 128, 8, 1089, True, 1088, 1088),
+    (32, 8, 128, 8, 1089, False, 320, 383),     # every key of the split of key tile 5, seen by all queries
+    (8, 2, 256, 8, 1089, True, 320, 383),
+    (32, 8, 128, 64, 8256, False, 7168, 8255),  # splits of many tiles: from the last eighth's first tile on
+    (32, 8, 128, 8, 1089, False, 0, 1088),      # no key with a score
+])
+def test_split_prefill_nan_split(orc, Hq, Hkv, D, S, N, f16, first, last):
+    """NaN in the K rows first..last of one kv head, so that every key a row
+    sees in one of the splits has a NaN score: no running maximum comes out of
+    such a split, but its NaN reaches the output, as in the oracle (fp16 outputs
+    hold an infinity for a NaN)."""
+    nan, h = 0x7E00 if f16 else 0x7FC0, 1
+
+    def old(k):
+        k[h, first:last + 1, 3] = nan
+
+    def new(k, v):
+        k[0, h, max(first - (N - S), 0):max(last + 1 - (N - S), 0), 3] = nan
+
+    mgr, ref = cached(orc, Hkv, D, N, S, 9000 + first, f16, plant=old)
+    got, want = chunk(orc, mgr, ref, Hq, Hkv, S, D, 9100 + first, f16, plant=new)
+    val = as_f16 if f16 else f32
+    G, seen = Hq // Hkv, np.arange(N - S, N) >= first
+    expect = np.zeros(want.shape, dtype=bool)
+    expect[:, h * G:(h + 1) * G, seen] = True
+    for x in (want, got):
+        assert np.array_equal(~np.isfinite(val(x)), expect)
+    assert np.array_equal(got[expect] & 0x7FFF, want[expect] & 0x7FFF)
+    fin = [np.where(expect, 0, x).astype(np.uint16) for x in (got, want)]
+    (assert_attn_close_f16 if f16 else assert_attn_close)(*fin, f"nan split D{D} N{N} keys {first}..{last}")
     mgr.close()
 
 
