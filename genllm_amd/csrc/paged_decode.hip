@@ -162,8 +162,8 @@ __device__ __forceinline__ void merge_last_arrival(const AttnParams& p, int h, f
             float bm = mw;
 #pragma unroll
             for (int u = 0; u < U; ++u) bm = fmaxf(bm, mv[u].x);
-            if (bm == -INFINITY) continue;  // nothing visible yet
-            const float a = mw == -INFINITY ? 0.0f : exp2_fast(mw - bm);
+            const float ref = bm == -INFINITY ? 0.0f : bm;
+            const float a = exp2_fast(mw - ref);  // 0 while mw = -inf
             lw *= a;
 #pragma unroll
             for (int hh = 0; hh < VH; ++hh) {
@@ -172,7 +172,7 @@ __device__ __forceinline__ void merge_last_arrival(const AttnParams& p, int h, f
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const float w = mv[u].x == -INFINITY ? 0.0f : exp2_fast(mv[u].x - bm);
+                const float w = exp2_fast(mv[u].x - ref);
                 lw += mv[u].y * w;
 #pragma unroll
                 for (int hh = 0; hh < VH; ++hh) {
@@ -641,16 +641,18 @@ __global__ __launch_bounds__(W * 64) void paged_decode_kernel(const int32_t* k_i
         float L = 0.0f, O0[VH], O1[VH];
 #pragma unroll
         for (int hh = 0; hh < VH; ++hh) O0[hh] = O1[hh] = 0.0f;
-        if (M != -INFINITY) {
+        // A wave without a maximum has weight 0, multiplied all the same: its l
+        // and o are zeros if the row sees none of its keys, NaN if every score
+        // is NaN.
+        const float ref = M == -INFINITY ? 0.0f : M;
 #pragma unroll
-            for (int w2 = w0; w2 < w0 + WP; ++w2) {
-                const float e = exp2_fast(lds_m[w2][ri] - M);
-                L += lds_l[w2][ri] * e;
+        for (int w2 = w0; w2 < w0 + WP; ++w2) {
+            const float e = exp2_fast(lds_m[w2][ri] - ref);
+            L += lds_l[w2][ri] * e;
 #pragma unroll
-                for (int hh = 0; hh < VH; ++hh) {
-                    O0[hh] += lds_o[w2][ri][128 * hh + 2 * lane] * e;
-                    O1[hh] += lds_o[w2][ri][128 * hh + 2 * lane + 1] * e;
-                }
+            for (int hh = 0; hh < VH; ++hh) {
+                O0[hh] += lds_o[w2][ri][128 * hh + 2 * lane] * e;
+                O1[hh] += lds_o[w2][ri][128 * hh + 2 * lane + 1] * e;
             }
         }
         if (p.n_splits == 1) {
@@ -709,6 +711,8 @@ __global__ __launch_bounds__(W * 64) void paged_decode_kernel(const int32_t* k_i
 // round trip for up to MW * kMergeU splits); the MW partials then meet in LDS
 // with the same rule
 //   M = max M_w, L = sum L_w 2^(M_w - M), O = sum O_w 2^(M_w - M), out = O / L.
+// (A split without a maximum has weight 0, which its l and o, NaN where every
+// score of the row is NaN, are multiplied by all the same.)
 // MW is 4, or 8 above 4 * kMergeU splits (measured: 8 waves cost about 0.4 us
 // at 31-32 splits and save 0.6 us at 103; 2 waves at 31 splits cost 0.3 us).  Blocks of 64 dims rather than one
 // workgroup per row (D dims) spread a row's partials over D / 64 CUs; on one
@@ -768,14 +772,14 @@ __global__ __launch_bounds__(MW * 64) void paged_decode_merge_kernel(const float
         float bm = mw;
 #pragma unroll
         for (int u = 0; u < U; ++u) bm = fmaxf(bm, mv[u].x);
-        if (bm == -INFINITY) continue;  // nothing visible yet
-        const float a = mw == -INFINITY ? 0.0f : exp2_fast(mw - bm);
+        const float ref = bm == -INFINITY ? 0.0f : bm;
+        const float a = exp2_fast(mw - ref);  // 0 while mw = -inf
         lw *= a;
 #pragma unroll
         for (int e = 0; e < PL; ++e) ow[e] *= a;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const float w = mv[u].x == -INFINITY ? 0.0f : exp2_fast(mv[u].x - bm);
+            const float w = exp2_fast(mv[u].x - ref);
             lw += mv[u].y * w;
 #pragma unroll
             for (int e = 0; e < PL; ++e) ow[e] += ov[u][e] * w;

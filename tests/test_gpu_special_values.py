@@ -119,3 +119,37 @@ def test_prefill_special_values(orc, S, N):
     assert np.array_equal(np.isnan(f32(want)), expected_nan_rows(q_abs, k_pos, v_pos))
     check(got, want, np.zeros_like(want, dtype=bool), f"prefill S{S} N{N}")
     ctx.close()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,S,N,pps,merge,heads,first,last", [
+    (16, 8, 128, 1, 993, 2, "kernel", 1, 992, 992),     # 32 splits, the last one of one key
+    (16, 8, 128, 1, 1000, 21, "kernel", 1, 336, 671),   # the middle one of 3 splits: alone in its merge wave
+    (16, 8, 128, 1, 1000, 21, "fused", 1, 336, 671),
+    (16, 8, 128, 1, 993, 2, "fused", 1, 992, 992),
+    (32, 8, 128, 1, 1000, 16, "kernel", 4, 512, 767),   # split workgroups of 4 kv heads
+    (16, 8, 128, 3, 994, 2, "kernel", 1, 992, 993),     # the first of three queries sees neither NaN key
+    (8, 2, 256, 1, 993, 2, "kernel", 1, 992, 992),
+    (8, 2, 256, 1, 1000, 21, "fused", 1, 336, 671),
+    (16, 8, 128, 1, 1000, 21, "kernel", 1, 0, 999),     # no key with a score
+])
+def test_decode_split_of_nan_keys(orc, Hq, Hkv, D, S, N, pps, merge, heads, first, last):
+    """NaN in the K rows first..last of one kv head, every key of one split
+    among them: the split finds no running maximum, and its NaN must still
+    reach the output through the workgroup's partial and the merge."""
+    ctx = Context(orc, Hkv, D, (N + 15) // 16 + 4, N, 8600 + N + first)
+    kt, _ = ctx.ref.page_table(0)
+    kp, h = ctx.ref.pool_array(0, 0), 1
+    for t in range(first, last + 1):
+        kp[kt[t // 16], t % 16, h, 5] = 0x7FC0
+    ctx.mgr.write_pool(0, 0, np.ascontiguousarray(kp))
+    q = synth.normal_bf16(8700 + N, (Hq, S, D))
+    got, _ = ctx.decode(q, pps=pps, merge=merge, heads=heads)
+    want = ctx.oracle(q)
+    expect = np.zeros(want.shape, dtype=bool)
+    expect[h * (Hq // Hkv):(h + 1) * (Hq // Hkv), np.arange(N - S, N) >= first] = True
+    assert np.array_equal(np.isnan(f32(want)), expect)
+    assert np.array_equal(np.isnan(f32(got)), expect)
+    assert np.all((got[expect] & 0x7FFF) == 0x7F81)
+    fin = [np.where(expect, 0, x).astype(np.uint16) for x in (got, want)]
+    assert_attn_close(*fin, f"nan split Hkv{Hkv} D{D} S{S} pps{pps} {merge} heads{heads}")
+    ctx.close()
