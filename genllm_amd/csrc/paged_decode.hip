@@ -870,9 +870,10 @@ int set_decode_tuning(int pages_per_split, int merge, int heads_per_wg) {
 // Heads per workgroup: kMultiHead where the one-head plan reaches
 // kMultiHeadMinPps pages per split (or where forced), for head_dim 128, kv
 // heads in groups of 4 and the merge kernel; else 1.
-// Short contexts run in one split (kOneSplitPages) unless the split size is
-// forced; the checks of the planned splits are made all the same, and *need is
-// the workspace they ask for.
+// Short contexts run in one split (kOneSplitPages) where every setting is
+// automatic: a forced split size, merge form, workgroup count or 4-head
+// workgroup keeps the planned splits.  The checks of the planned splits are
+// made all the same, and *need is the workspace they ask for.
 int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws, size_t* need_out) {
     if (need_out) *need_out = 0;
     if (p.G * p.S > kRows) return fail(GENLLM_ERR_INVALID, "paged decode: seq_len * groups must be <= 16");
@@ -881,10 +882,11 @@ int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws, size_t* need_ou
     int pps = cfg.pps.load(std::memory_order_relaxed);
     const int heads = cfg.heads.load(std::memory_order_relaxed);
     const int cus = device_cu_count();
-    const bool multi_ok =
-        D == 128 && p.Hkv % kMultiHead == 0 && cfg.merge.load(std::memory_order_relaxed) == kDecodeMergeKernel;
+    const int merge = cfg.merge.load(std::memory_order_relaxed);
+    const double wg_per_cu = cfg.wg_per_cu.load(std::memory_order_relaxed);
+    const bool multi_ok = D == 128 && p.Hkv % kMultiHead == 0 && merge == kDecodeMergeKernel;
     if (pps <= 0) {
-        const int64_t target = std::max<int64_t>(1, int64_t(cfg.wg_per_cu.load(std::memory_order_relaxed) * cus));
+        const int64_t target = std::max<int64_t>(1, int64_t(wg_per_cu * cus));
         pps = int((int64_t(p.n_pages) * p.Hkv + target - 1) / target);
         if (pps < 2) pps = 2;
         // long ranges: kMultiHead kv heads per workgroup, the same workgroup count
@@ -909,15 +911,15 @@ int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws, size_t* need_ou
             return fail(GENLLM_ERR_INVALID, "paged decode: workspace too small (need " + std::to_string(need) +
                                                 " bytes, have " + std::to_string(ws_bytes) + ")");
         if (need_out) *need_out = need;
-        if (cfg.pps.load(std::memory_order_relaxed) <= 0 &&
-            p.n_pages <= (D == 128 ? kOneSplitPages<128> : kOneSplitPages<256>)) {
+        const bool automatic = cfg.pps.load(std::memory_order_relaxed) <= 0 && merge == kDecodeMergeKernel &&
+                               p.heads_per_wg == 1 && wg_per_cu == 1.0;
+        if (automatic && p.n_pages <= (D == 128 ? kOneSplitPages<128> : kOneSplitPages<256>)) {
             p.pages_per_split = p.n_pages;
             p.n_splits = 1;
-            p.heads_per_wg = 1;
             return GENLLM_OK;
         }
         p.partial = reinterpret_cast<float*>(static_cast<char*>(ws) + kDecodeCounterBytes);
-        if (cfg.merge.load(std::memory_order_relaxed) == kDecodeMergeFused) p.counters = static_cast<int32_t*>(ws);
+        if (merge == kDecodeMergeFused) p.counters = static_cast<int32_t*>(ws);
     }
     return GENLLM_OK;
 }

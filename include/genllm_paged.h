@@ -265,8 +265,8 @@ int genllm_paged_decode(const void *q, int64_t q_head_stride, int64_t q_tok_stri
 /* No counterpart in the reference: a tuning and test hook for the decode
  * kernels of this library (genllm_paged_decode, _noalloc, the op and its
  * device-position steps), process-wide, for later calls.  pages_per_split > 0
- * forces the split size (0: automatic, about one workgroup per CU, one split
- * for a few pages).  merge:
+ * forces the split size (0: automatic, about one workgroup per CU, and one
+ * split for a few pages unless merge 1 or 4 heads are asked for).  merge:
  * 0 = a merge kernel after the split kernel (default), 1 = the last split
  * workgroup of each kv head to finish merges it in the same launch.
  * heads_per_workgroup: kv heads one split workgroup reads; 0 = automatic (4

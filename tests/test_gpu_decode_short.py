@@ -29,6 +29,20 @@ def test_short_decode_vs_oracle(orc, Hkv, G, D, S, N, causal):
     ctx.close()
 
 
+@pytest.mark.parametrize("merge,heads,split", [("kernel", 4, True), ("fused", 0, True), ("kernel", 1, False), ("kernel", 0, False)])
+def test_short_decode_takes_forced_settings(orc, merge, heads, split):
+    """A forced merge form or 4 kv heads per workgroup keep the planned splits
+    of a short context (their partials are in the workspace, past its 1 KiB of
+    counters); the automatic plan, and one head, leave the workspace alone."""
+    N = 64
+    ctx = Context(orc, 8, 128, 8, N, 8850)
+    q = synth.normal_bf16(8950, (32, 1, 128))
+    got, ws = ctx.decode(q, merge=merge, heads=heads)
+    assert_attn_close(got, ctx.oracle(q), f"forced {merge} heads{heads}")
+    assert bool(ws[1024:].any()) == split
+    ctx.close()
+
+
 @pytest.mark.parametrize("N", [100, 300])
 def test_short_decode_keeps_its_workspace_check(N):
     q = paged.to_device_bf16(synth.normal_bf16(1, (8, 1, 128)))

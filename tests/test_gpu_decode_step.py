@@ -184,7 +184,8 @@ def test_captured_36_layer_step_replays_20_tokens(orc):
     st.close()
 
 
-def test_partial_window_sync_and_exhaustion(orc):
+@pytest.mark.parametrize("pps", [0, 2])  # 2: several splits, and the merge kernel of a refused step
+def test_partial_window_sync_and_exhaustion(orc, pps):
     """A window staged for 40 tokens of which 5 run: sync gives the 3 unused
     pages back so that later host appends hand out the reference's ids; a
     window of 3 replayed 4 times: the 4th step does nothing and sync reports
@@ -200,7 +201,7 @@ def test_partial_window_sync_and_exhaustion(orc):
                               buf.out[0], Hq // Hkv, scale_for(D))
     assert e.value.code == ERR_INVALID
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    with paged.decode_tuned(pps), torch.cuda.graph(g):
         for l in range(L):
             buf.layer_step(st, l, rope=False)
     run_checked_replays(st, buf, g, 5, P, seed=8000, rope=False)
@@ -255,17 +256,17 @@ def test_step_head_dim_256_across_8192(orc):
     (32, 8, 128, 1, 200, 128, "fused"),  # single-launch merge: no merge kernel either
     (8, 2, 256, 1, 90, 64, None),       # Qwen3.5: RoPE on the first 64 of 256 dims
     (16, 8, 128, 2, 40, 128, "heads4"),  # split workgroups reading 4 kv heads each, steps crossing pages
+    (16, 8, 128, 2, 300, 128, "split2"),  # 11 splits: the merge kernel advances the position
+    (16, 8, 128, 2, 300, 128, "split2 heads4"),
 ])
 def test_step_variants(orc, request, Hq, Hkv, D, S, P, rope_dim, merge):
     """Device-position steps beyond the single-token default plan: the query
     chunk, the split plan, the merge form and the rotary width change, and
     every replay still matches the oracle run with host positions (RoPE'd q
     bit-exact, attention within tolerance, pools bit-exact)."""
-    if merge == "heads4":
-        paged.decode_tuning(0, "kernel", 4)
-        request.addfinalizer(lambda: paged.decode_tuning(0, "kernel"))
-    elif merge:
-        paged.decode_tuning(0, merge)
+    tuning = {"heads4": (0, "kernel", 4), "fused": (0, "fused"), "split2": (2,), "split2 heads4": (2, "kernel", 4)}
+    if merge:
+        paged.decode_tuning(*tuning[merge])
         request.addfinalizer(lambda: paged.decode_tuning(0, "kernel"))
     G, L, steps, max_seq = Hq // Hkv, 2, 8, 512
     pool = (P + S * steps + 15) // 16 + 2

@@ -202,7 +202,8 @@ def test_fill_normal_f16_matches_host_formula():
     assert abs(want.mean()) < 0.02 and abs(want.std() - 1) < 0.02
 
 
-@pytest.mark.parametrize("P,steps,merge", [(40, 12, "kernel"), (200, 6, "fused"), (40, 12, "heads4")])
+@pytest.mark.parametrize("P,steps,merge", [(40, 12, "kernel"), (200, 6, "fused"), (40, 12, "heads4"),
+                                           (300, 6, "split2"), (300, 6, "split2 heads4")])
 def test_f16_device_position_step(orc, request, P, steps, merge):
     """fp16 layers through the device-position decode step: the step staged
     (genllm_kv_stage_decode), genllm_paged_attention_step captured once into a
@@ -210,11 +211,10 @@ def test_f16_device_position_step(orc, request, P, steps, merge):
     the single-launch merge), each replay against the oracle's fp16 path at the
     host position, pools bit-exact; after genllm_kv_sync_decode the host page
     table and num_cached equal the oracle's."""
-    if merge == "heads4":  # split workgroups reading 4 kv heads each
-        paged.decode_tuning(0, "kernel", 4)
-        request.addfinalizer(lambda: paged.decode_tuning(0, "kernel"))
-    elif merge != "kernel":
-        paged.decode_tuning(0, merge)
+    # heads4: split workgroups reading 4 kv heads each; split2: splits of 2 pages
+    tuning = {"heads4": (0, "kernel", 4), "fused": (0, "fused"), "split2": (2,), "split2 heads4": (2, "kernel", 4)}
+    if merge != "kernel":
+        paged.decode_tuning(*tuning[merge])
         request.addfinalizer(lambda: paged.decode_tuning(0, "kernel"))
     Hq, Hkv, D = 32, 8, 128
     G, pool = Hq // Hkv, (P + steps + 15) // 16 + 3
