@@ -439,7 +439,9 @@ extern "C" int genllm_kv_reserve_layer(genllm_kv* kv, int32_t layer, int32_t max
     // a captured device-position step holds the current buffer's address.
     // Checked first, so that a refusal changes nothing.
     const int rows = 16;  // decode kernel limit: (query, q-head) rows per kv head
-    const size_t ws_need = decode_workspace_bytes(rows * s.n_kv_heads, s.n_kv_heads, 1, s.head_dim, max_blocks);
+    // two splits at least: an out over the inputs takes them on one page as well
+    const size_t ws_need =
+        decode_workspace_bytes(rows * s.n_kv_heads, s.n_kv_heads, 1, s.head_dim, std::max(max_blocks, 2));
     if (ws_need > kv->ws_bytes)
         for (const auto& kvp : kv->layers)
             if (kvp.second.active && kvp.second.staged)
@@ -700,6 +702,7 @@ extern "C" int genllm_paged_attention(genllm_kv* kv, int32_t layer, const void* 
     if (int rc = op_params(*s, q, k, v, out, batch, n_q_heads, seq_len, head_dim, n_kv_heads, n_kv_groups, scale,
                            causal, n_after, p))
         return rc;
+    fuse_append(p, *s, k, v, seq_len, head_dim, pos0);
     if (int rc = prepare_attention(p, head_dim, kv)) return rc;
 
     // 1. append (append_kv_from_tensor, attention.cpp:146): head-major [Hkv][S][D].
@@ -713,7 +716,6 @@ extern "C" int genllm_paged_attention(genllm_kv* kv, int32_t layer, const void* 
     pa.max_blocks = s->max_blocks;
 
     // 2. attend over all cached tokens
-    fuse_append(p, *s, k, v, seq_len, head_dim, pos0);
     if (fuse) {
         // seq_len <= 16 opens at most 2 pages, which fit the launch arguments
         // (append_pages put them in pa.upd, as it holds up to 256)
@@ -856,8 +858,8 @@ extern "C" int genllm_paged_attention_step(genllm_kv* kv, int32_t layer, const v
                            causal, window_end, p))
         return rc;
     p.step = s->d_step;
-    if (int rc = prepare_attention(p, head_dim, kv)) return rc;
     fuse_append(p, *s, k, v, seq_len, head_dim, 0);
+    if (int rc = prepare_attention(p, head_dim, kv)) return rc;
     return launch_attention(p, *s, head_dim, as_stream(stream));
 }
 

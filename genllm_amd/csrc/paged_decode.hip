@@ -865,6 +865,29 @@ int set_decode_tuning(int pages_per_split, int merge, int heads_per_wg) {
     return GENLLM_OK;
 }
 
+namespace {
+// Whether out overlaps rows that another workgroup of the split kernel may
+// still read: the appended K/V rows, or q, unless out is q itself (a workgroup
+// writes the rows of its own kv heads, which no other one reads).
+bool out_over_inputs(const AttnParams& p, int D) {
+    const auto bytes = [&](int64_t heads, int64_t head_stride, int64_t tok_stride) {
+        return size_t(((heads - 1) * head_stride + (p.S - 1) * tok_stride + D) * 2);
+    };
+    const uintptr_t o = reinterpret_cast<uintptr_t>(p.out);
+    const size_t o_bytes = bytes(p.Hq, p.o_head_stride, p.o_tok_stride);
+    const auto meets = [&](const uint16_t* x, size_t n) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(x);
+        return o < a + n && a < o + o_bytes;
+    };
+    if (p.k_new) {
+        const size_t n = bytes(p.Hkv, p.new_head_stride, p.new_tok_stride);
+        if (meets(p.k_new, n) || meets(p.v_new, n)) return true;
+    }
+    const bool in_place = p.out == p.q && p.o_head_stride == p.q_head_stride && p.o_tok_stride == p.q_tok_stride;
+    return !in_place && meets(p.q, bytes(p.Hq, p.q_head_stride, p.q_tok_stride));
+}
+}  // namespace
+
 // Pages per split: about wg_per_cu (default 1) workgroups per CU over all kv
 // heads, at most 256 splits (a forced value, genllm_decode_tuning, wins).
 // Heads per workgroup: kMultiHead where the one-head plan reaches
@@ -873,7 +896,10 @@ int set_decode_tuning(int pages_per_split, int merge, int heads_per_wg) {
 // Short contexts run in one split (kOneSplitPages) where every setting is
 // automatic: a forced split size, merge form, workgroup count or 4-head
 // workgroup keeps the planned splits.  The checks of the planned splits are
-// made all the same, and *need is the workspace they ask for.
+// made all the same, and *need is the workspace they ask for.  An out over the
+// inputs is written by the merge kernel, after every split workgroup has ended:
+// the planned splits stay, and where the op would plan one (k_new), a second,
+// empty one brings that kernel in.
 int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws, size_t* need_out) {
     if (need_out) *need_out = 0;
     if (p.G * p.S > kRows) return fail(GENLLM_ERR_INVALID, "paged decode: seq_len * groups must be <= 16");
@@ -902,6 +928,11 @@ int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws, size_t* need_ou
     p.n_splits = (p.n_pages + pps - 1) / pps;
     p.partial = nullptr;
     p.counters = nullptr;
+    const bool late_out = out_over_inputs(p, D);
+    if (late_out && p.k_new && p.n_splits == 1 && p.Hkv <= kDecodeMaxKvHeads) {
+        p.pages_per_split = p.n_pages;
+        p.n_splits = 2;
+    }
     if (p.n_splits > 1) {
         if (p.Hkv > kDecodeMaxKvHeads)
             return fail(GENLLM_ERR_UNSUPPORTED, "paged decode: at most 256 kv heads");
@@ -912,14 +943,14 @@ int decode_plan(AttnParams& p, int D, size_t ws_bytes, void* ws, size_t* need_ou
                                                 " bytes, have " + std::to_string(ws_bytes) + ")");
         if (need_out) *need_out = need;
         const bool automatic = cfg.pps.load(std::memory_order_relaxed) <= 0 && merge == kDecodeMergeKernel &&
-                               p.heads_per_wg == 1 && wg_per_cu == 1.0;
+                               p.heads_per_wg == 1 && wg_per_cu == 1.0 && !late_out;
         if (automatic && p.n_pages <= (D == 128 ? kOneSplitPages<128> : kOneSplitPages<256>)) {
             p.pages_per_split = p.n_pages;
             p.n_splits = 1;
             return GENLLM_OK;
         }
         p.partial = reinterpret_cast<float*>(static_cast<char*>(ws) + kDecodeCounterBytes);
-        if (merge == kDecodeMergeFused) p.counters = static_cast<int32_t*>(ws);
+        if (merge == kDecodeMergeFused && !late_out) p.counters = static_cast<int32_t*>(ws);
     }
     return GENLLM_OK;
 }

@@ -140,8 +140,8 @@ int genllm_kv_block_free(genllm_kv *kv, int32_t layer, int32_t which, int32_t id
  * attention.cu:511).  Chunks of up to 16 (query, q-head) rows per kv head run
  * the split-K decode kernel, longer chunks the MFMA prefill kernels, with the
  * keys split over workgroups where the chunk alone would leave the GPU idle.
- * k and v are read while out is written in the decode kernel's range; longer
- * chunks take an out that overlaps them as well.  Every
+ * out may overlap k and v, and may be q (the same address); a short chunk then
+ * writes it in a second kernel.  Every
  * argument check and the split plan run before the layer changes: a call that
  * returns an error leaves num_cached, the page tables and the block pools as
  * they were. */

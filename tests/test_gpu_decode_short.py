@@ -1,14 +1,17 @@
 """Decode over contexts of a few pages: up to kOneSplitPages pages (12 at
 head_dim 128, 5 at 256) one split writes the output itself, above that the
 planned splits and their merge.  Both sides of the line against the oracle,
-and a workspace too small for the planned splits is refused on both."""
+a workspace too small for the planned splits is refused on both, and an output
+over the inputs is written only after every workgroup has read them."""
 import numpy as np
 import pytest
+import torch
 
 from genllm_amd import paged, synth
 from genllm_amd._lib import ERR_INVALID, GenllmError
 from helpers import assert_attn_close, scale_for
 from test_gpu_decode import Context
+from test_gpu_f16_batch import check_pools, make
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +55,45 @@ def test_short_decode_keeps_its_workspace_check(N):
     with pytest.raises(GenllmError) as e:
         paged.paged_decode(q, q.clone(), pool, pool, ids, ids, (N + 15) // 16, N, 2, scale_for(128), small)
     assert e.value.code == ERR_INVALID and "workspace too small" in str(e.value)
+
+
+@pytest.mark.parametrize("step", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,D,S,N,over,merge", [
+    (32, 8, 128, 1, 100, "k", "kernel"),  # 7 pages: one split but for the overlap
+    (32, 8, 128, 1, 100, "v", "kernel"),
+    (32, 8, 128, 1, 100, "q", "kernel"),  # a head further on in the same buffer
+    (32, 8, 128, 2, 20, "k", "kernel"),   # 2 pages: one split is planned
+    (16, 8, 128, 1, 5, "v", "fused"),     # one page
+    (32, 8, 128, 1, 300, "k", "fused"),   # several splits
+    (8, 2, 256, 1, 70, "v", "kernel"),
+])
+def test_decode_output_over_inputs(orc, Hq, Hkv, D, S, N, over, merge, step):
+    """The op and its device-position step with the new K or V rows inside the
+    output buffer, and with an output that starts one head before q: outputs
+    and pools as with separate buffers."""
+    mgr, ref = make(orc, Hkv, D, (N + 15) // 16, 9300 + N, orc.BF16)
+    k, v = (synth.normal_bf16(9310 + N + i, (Hkv, N - S, D)) for i in (0, 1))
+    mgr.append_kv_from_pos(0, paged.to_device_bf16(k), paged.to_device_bf16(v), 0)
+    ref.append_kv_from_pos(0, k, v, 0)
+    q, k, v = (synth.normal_bf16(9320 + N + i, (1, h, S, D)) for i, h in enumerate((Hq, Hkv, Hkv)))
+    want, rc = ref.paged_attention(0, q, k, v, Hq // Hkv, scale_for(D), True)
+    assert rc == 0
+    buf = torch.zeros((1, Hq + 1, S, D), dtype=torch.bfloat16, device="cuda")
+    out, qd, kd, vd = buf[:, :Hq], paged.to_device_bf16(q), paged.to_device_bf16(k), paged.to_device_bf16(v)
+    if over == "q":
+        qd = buf[:, 1:].copy_(qd)
+    elif over == "k":
+        kd = buf[:, Hq - Hkv:Hq].copy_(kd)
+    else:
+        vd = buf[:, Hq - Hkv:Hq].copy_(vd)
+    with paged.decode_tuned(0, merge):
+        if step:
+            mgr.stage_decode(0, S)
+            paged.paged_attention_step(mgr, 0, qd, kd, vd, out, Hq // Hkv, scale_for(D))
+            assert mgr.sync_decode(0) == N
+        else:
+            paged.paged_attention(mgr, 0, qd, kd, vd, out, Hq // Hkv, scale_for(D))
+    torch.cuda.synchronize()
+    assert_attn_close(paged.to_host_bits(out), want, f"out over {over} D{D} S{S} N{N} {merge} step {step}")
+    check_pools(mgr, ref, f"out over {over}")
+    mgr.close()
