@@ -920,13 +920,37 @@ int prefill_splits(int64_t units, int64_t rows, int n_cached, int head_dim, size
     return best;
 }
 
+// Whether out overlaps the rows of a batch (out that is q itself aside: a
+// workgroup writes the rows it read).  An entry's output may then lie over
+// another entry's inputs, which is sound only one entry after another.
+static bool out_over_entries(const AttnParams& p, const PrefillBatch& b, int head_dim) {
+    if (b.n <= 1) return false;
+    const auto bytes = [&](int64_t stride, int64_t heads, int64_t head_stride, int64_t tok_stride) {
+        return size_t(((b.n - 1) * stride + (heads - 1) * head_stride + (p.S - 1) * tok_stride + head_dim) * 2);
+    };
+    const uintptr_t o = reinterpret_cast<uintptr_t>(p.out);
+    const size_t o_bytes = bytes(b.o_stride, p.Hq, p.o_head_stride, p.o_tok_stride);
+    const auto meets = [&](const uint16_t* x, size_t n) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(x);
+        return o < a + n && a < o + o_bytes;
+    };
+    const bool in_place = p.out == p.q && b.o_stride == b.q_stride && p.o_head_stride == p.q_head_stride &&
+                          p.o_tok_stride == p.q_tok_stride;
+    if (!in_place && meets(p.q, bytes(b.q_stride, p.Hq, p.q_head_stride, p.q_tok_stride))) return true;
+    if (b.kv_stride == 0) return false;  // the pages of a cache
+    const size_t kv = bytes(b.kv_stride, p.Hkv, p.kv_head_stride, p.kv_row);
+    return meets(p.k_pool, kv) || meets(p.v_pool, kv);
+}
+
 int launch_paged_prefill(const AttnParams& p, int head_dim, hipStream_t stream, const PrefillBatch& b, float* ws,
                          size_t ws_bytes, const PrefillAppend* append) {
     if (head_dim != 128 && head_dim != 256) return fail(GENLLM_ERR_UNSUPPORTED, "paged prefill: head_dim must be 128 or 256");
     if (p.S <= 0 || p.n_pages <= 0 || b.n <= 0) return GENLLM_OK;
     const int64_t rows = int64_t(p.S) * p.G;
     // entries per launch: a grid of about 2^21 workgroups at most (HIP takes up to 2^32 threads)
-    const int64_t per = std::max<int64_t>(1, (int64_t(1) << 21) / ((rows + QT - 1) / QT * p.Hkv));
+    const int64_t per = out_over_entries(p, b, head_dim)
+                            ? 1
+                            : std::max<int64_t>(1, (int64_t(1) << 21) / ((rows + QT - 1) / QT * p.Hkv));
     for (int64_t b0 = 0; b0 < b.n; b0 += per) {
         AttnParams pb = p;
         pb.q += b0 * b.q_stride;

@@ -139,6 +139,42 @@ def test_flash_batch_in_one_launch(orc, B, Hq, Hkv, S, D):
     assert_attn_close(paged.to_host_bits(out), orc.flash_attention(q, k, v, Hq // Hkv, scale_for(D), True), f"flash B{B}")
 
 
+@pytest.mark.parametrize("Hq,Hkv,S,D,over", [
+    (4, 4, 70, 128, "q"),
+    (4, 4, 70, 128, "k"),
+    (4, 4, 33, 256, "v"),
+    (2, 2, 300, 128, "q"),
+])
+def test_flash_batch_output_over_earlier_inputs(orc, Hq, Hkv, S, D, over):
+    """Each entry's output over the q, k or v rows of the entry before it:
+    right as long as the entries run one after another."""
+    B = 4
+    q, k, v = (synth.normal_bf16(7100 + i, (B, h, S, D)) for i, h in enumerate((Hq, Hkv, Hkv)))
+    d = {"q": paged.to_device_bf16(q), "k": paged.to_device_bf16(k), "v": paged.to_device_bf16(v)}
+    buf = torch.zeros((B + 1, Hq, S, D), dtype=torch.bfloat16, device="cuda")
+    d[over] = buf[1:].copy_(d[over])
+    paged.flash_attention(d["q"], d["k"], d["v"], buf[:B], Hq // Hkv, scale_for(D))
+    torch.cuda.synchronize()
+    want = orc.flash_attention(q, k, v, Hq // Hkv, scale_for(D), True)
+    assert_attn_close(paged.to_host_bits(buf[:B]), want, f"flash out over {over}")
+
+
+def test_op_batch_output_over_earlier_queries(orc):
+    """The op's prefill chunk with each entry's output over the queries of the
+    entry before it."""
+    B, Hq, Hkv, D, S, N = 3, 4, 2, 128, 40, 200
+    mgr, ref = cached(orc, Hkv, D, N, S, 7200, False)
+    q, k, v = (synth.normal_bf16(7210 + i, (B, h, S, D)) for i, h in enumerate((Hq, Hkv, Hkv)))
+    buf = torch.zeros((B + 1, Hq, S, D), dtype=torch.bfloat16, device="cuda")
+    qd = buf[1:].copy_(paged.to_device_bf16(q))
+    paged.paged_attention(mgr, 0, qd, paged.to_device_bf16(k), paged.to_device_bf16(v), buf[:B], Hq // Hkv, scale_for(D))
+    torch.cuda.synchronize()
+    want, rc = ref.paged_attention(0, q, k, v, Hq // Hkv, scale_for(D), True)
+    assert rc == 0
+    assert_attn_close(paged.to_host_bits(buf[:B]), want, "op out over q")
+    mgr.close()
+
+
 @pytest.mark.parametrize("Hq,Hkv,S,N,causal", [
     (4, 2, 33, 1280, True),   # 10 whole 128-key tiles
     (2, 1, 20, 1281, True),   # the last key alone in its tile
