@@ -871,14 +871,35 @@ int launch_prefill(const AttnParams& p, const PrefillGrid& gr, const AppendArg<k
 
 int resident_workgroups(int head_dim) { return device_cu_count() * (head_dim == 128 ? 2 : 1); }
 
+// The terms of prefill_splits' estimate.
+struct SplitCost {
+    double tile_us, split_tile_us;  // a 64-key tile in the unsplit kernel, in the split kernel
+    static constexpr double kPairTileUs = 1.25;  // ... with two workgroups on a CU
+    static constexpr double kMergeUs = 6.0, kMergeUsPerMB = 0.46;
+    static constexpr double kUnsplit = 0.85;  // less where the keys are still in the caches
+    explicit SplitCost(int head_dim) : tile_us(head_dim == 128 ? 0.8 : 1.45), split_tile_us(head_dim == 128 ? 0.85 : 1.45) {}
+    double unsplit(int64_t tiles) const { return kUnsplit * double(tiles) * tile_us; }
+};
+
 }  // namespace
 
-// Every split launch keeps its workgroups resident at once, 64 rows each, so
-// its partials fit this whatever its shape (17 MB at either head_dim).  A
-// cache of up to 4 key tiles is never split.
+// The most partials any chunk of a layer of max_tokens may hand over: every
+// split launch keeps its workgroups resident at once, 64 rows each (17 MB at
+// either head_dim), and over few keys only launches whose merge costs less than
+// the split saves are split (none up to 10 key tiles at head_dim 128, 6 at 256;
+// the whole 17 MB from 22 and 13 tiles on).
 size_t prefill_workspace_bytes(int head_dim, int64_t max_tokens) {
-    if ((head_dim != 128 && head_dim != 256) || max_tokens <= 256) return 0;
-    return size_t(resident_workgroups(head_dim)) * QT * (head_dim + 2) * sizeof(float);
+    if (head_dim != 128 && head_dim != 256) return 0;
+    const SplitCost cost(head_dim);
+    const double cap = double(resident_workgroups(head_dim)) * QT * (head_dim + 2) * sizeof(float);
+    double most = 0.0;
+    const int64_t last = (max_tokens + 63) / 64;
+    for (int64_t tiles = 2; tiles <= last && most < cap; ++tiles)
+        for (int64_t ns = 2; ns <= std::min<int64_t>(tiles, kMaxPrefillSplits); ++ns) {
+            const double gain = cost.unsplit(tiles) - double((tiles + ns - 1) / ns) * cost.split_tile_us - cost.kMergeUs;
+            most = std::max(most, std::min(gain / cost.kMergeUsPerMB * 1e6, cap));
+        }
+    return size_t(most);
 }
 
 // Key splits of a launch of `rows` rows for each of `units` (batch entry, kv
@@ -886,7 +907,7 @@ size_t prefill_workspace_bytes(int head_dim, int64_t max_tokens) {
 // workgroups are all resident at once.  Unsplit, a chunk of few rows leaves
 // most CUs idle while each of its workgroups walks all key tiles in turn.
 // Estimate, in us (fitted to kernel traces on MI355X): a workgroup's longest
-// chain of 64-key tiles at kTileUs each (kSplitTileUs in the split kernel, or
+// chain of 64-key tiles at tile_us each (split_tile_us in the split kernel, or
 // kPairTileUs where two workgroups share a CU), and for a split launch the
 // hand-over and the merge kernel, kMergeUs plus kMergeUsPerMB of partials
 // written and read back.  Measured, both kernels against one unsplit 8-wave
@@ -901,20 +922,17 @@ size_t prefill_workspace_bytes(int head_dim, int64_t max_tokens) {
 //   8/2,  256, 128 of 1128: 18.5 against  29.8 us (6)
 //   8/2,  256,  64 of 8192: 24.0 against 186.2 us (26)
 int prefill_splits(int64_t units, int64_t rows, int n_cached, int head_dim, size_t ws_bytes) {
-    const bool d128 = head_dim == 128;
-    const double kTileUs = d128 ? 0.8 : 1.45, kSplitTileUs = d128 ? 0.85 : 1.45, kPairTileUs = 1.25;
-    const double kMergeUs = 6.0, kMergeUsPerMB = 0.46;
-    const double kUnsplit = 0.85;  // less where the keys are still in the caches
+    const SplitCost cost(head_dim);
     const int64_t cus = device_cu_count(), wgs = (rows + QT - 1) / QT * units;
     const int64_t tiles = (int64_t(n_cached) + 63) / 64;
     const int64_t most = std::min<int64_t>({resident_workgroups(head_dim) / wgs, tiles, kMaxPrefillSplits});
     int best = 1;
-    double best_us = kUnsplit * double(tiles) * kTileUs;
+    double best_us = cost.unsplit(tiles);
     for (int64_t ns = 2; ns <= most; ++ns) {
         const double bytes = double(ns * units * rows) * (head_dim + 2) * sizeof(float);
         if (bytes > double(ws_bytes)) break;
-        const double us = double((tiles + ns - 1) / ns) * (wgs * ns <= cus ? kSplitTileUs : kPairTileUs) + kMergeUs +
-                          bytes * 1e-6 * kMergeUsPerMB;
+        const double us = double((tiles + ns - 1) / ns) * (wgs * ns <= cus ? cost.split_tile_us : cost.kPairTileUs) +
+                          cost.kMergeUs + bytes * 1e-6 * cost.kMergeUsPerMB;
         if (us < best_us) best = int(ns), best_us = us;
     }
     return best;

@@ -63,10 +63,14 @@ int genllm_kv_init_layer(genllm_kv *kv, int32_t layer, int32_t n_kv_heads, int32
  * kv_cache pool -- exactly the 2 * max_blocks * block_bytes per layer the
  * reference scheduler sizes it for (scheduler.cpp:62-79, 371).  The device
  * page table (max_blocks entries), its pinned host staging, the manager's
- * decode workspace and, for more than 256 tokens, the layer's scratch for
- * prefill chunks whose keys are split over workgroups (17 MB; without memory
- * for it the chunks run unsplit) are allocated separately, here, once: the op
- * itself never allocates, frees or synchronises. */
+ * decode workspace and, for more than 640 tokens (384 at head_dim 256), the
+ * layer's scratch for prefill chunks whose keys are split over workgroups are
+ * allocated separately, here, once: the op itself never allocates, frees or
+ * synchronises.  The scratch is sized for the largest plan the layer can make,
+ * 17 MB from 1345 (769) tokens on: 0.6 GB over 36 layers, next to the kv_cache
+ * pool.  Where that memory is not left the call succeeds all the same and the
+ * layer's chunks run unsplit, up to several times slower for a short chunk
+ * over a long cache. */
 int genllm_kv_reserve_layer(genllm_kv *kv, int32_t layer, int32_t max_blocks);
 /* PagedAttentionManager::is_active, page_attention.h:82-85; *active = 0/1 */
 int genllm_kv_is_active(genllm_kv *kv, int32_t layer, int32_t *active);

@@ -124,6 +124,21 @@ def test_split_prefill_nan_split(orc, Hq, Hkv, D, S, N, f16, first, last):
     mgr.close()
 
 
+@pytest.mark.parametrize("D,tokens,most", [(128, 640, 0), (128, 1024, 9), (256, 384, 0)])
+def test_split_scratch_fits_the_layer(D, tokens, most):
+    """A layer whose chunks are never split reserves no scratch for it, one with
+    few tokens what its largest plan needs (MB, on top of the page table and
+    the decode workspace, which take less than 5 MB with their 2 MB pages)."""
+    mgr = paged.PagedAttentionManager(2 * tokens * D * 2 + (1 << 20))
+    mgr.init_layer(0, 1, D)
+    free = torch.cuda.mem_get_info()[0]
+    mgr.reserve_layer(0, tokens // 16)
+    used = (free - torch.cuda.mem_get_info()[0]) / 1e6
+    print(f"D{D} {tokens} tokens: {used:.1f} MB", flush=True)
+    assert used <= most + 5
+    mgr.close()
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,S,D", [
     (3, 4, 2, 70, 128),   # the q heads of a kv head packed into row tiles
     (5, 2, 1, 1, 256),
