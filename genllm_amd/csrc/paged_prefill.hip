@@ -71,23 +71,31 @@ constexpr int kMaxPrefillSplits = 32;
 // division takes about thirty (17 queries of 17 keys, 16 q / 8 kv heads: 5.8 ->
 // 5.4 us; 300 of 2000: 21.2 -> 20.3 us).
 struct FastDiv {
-    uint32_t m = 1, s1 = 0, s2 = 0;
+    uint32_t m = 1;
+    uint16_t s1 = 0, s2 = 0;
     FastDiv() = default;
     explicit FastDiv(uint32_t d) {
         uint32_t l = 0;
         while (l < 32 && (uint64_t(1) << l) < d) ++l;
         m = uint32_t(((uint64_t(1) << 32) * ((uint64_t(1) << l) - d)) / d + 1);
-        s1 = l ? 1 : 0;
-        s2 = l ? l - 1 : 0;
+        s1 = uint16_t(l ? 1 : 0);
+        s2 = uint16_t(l ? l - 1 : 0);
     }
     __device__ __forceinline__ int operator()(int x) const {
         const uint32_t t = __umulhi(m, uint32_t(x));
-        return int((t + ((uint32_t(x) - t) >> s1)) >> s2);
+        return int((t + ((uint32_t(x) - t) >> uint32_t(s1))) >> uint32_t(s2));
     }
 };
 
 // What a launch adds to the attention parameters: batch entries (element
-// strides between them) and the key splits.
+// strides between them) and the key splits.  The kernels take it ahead of
+// AttnParams, in this order, so that what the prologue reads of both lies in
+// the first four 64-byte lines of the argument block: every line is fetched
+// anew in each launch, and with the fields spread over six of them, or held in
+// scalar registers through the tile loop, a launch took 0.3-0.5 us longer
+// (late_args; both: 16 q / 8 kv heads, 1700 tokens 24.0 against 24.7 us, 2048
+// tokens 29.0 against 29.4; 8 / 2 heads of 256, 2048 tokens 42.7 against 43.5;
+// medians of three traces each, taken in turn).
 struct PrefillGrid {
     int64_t q_batch = 0, o_batch = 0, kv_batch = 0;
     int32_t batch = 1, n_splits = 1;
@@ -95,8 +103,8 @@ struct PrefillGrid {
     int32_t pack = 1;          // q heads whose rows share row tiles: the groups of a kv head, or 1
     int32_t units = 1;         // batch entries x (q heads / pack)
     // pack, units, q heads / pack, groups / pack, kv heads, n_splits
-    FastDiv by_pack, by_units, by_heads, by_groups, by_hkv, by_splits;
-    int32_t n_rt = 0;                           // row tiles of a kv head
+    int32_t n_rt = 0;          // row tiles of a unit
+    FastDiv by_units, by_heads, by_groups, by_pack, by_splits, by_hkv;
     float* partial = nullptr;  // n_splits > 1: o [split][unit][row][D], then {m, l} [split][unit][row]
 };
 
@@ -206,21 +214,22 @@ __device__ __forceinline__ void prefill_exact_part(const AttnParams& p, const ui
     res[4 * DB + 1] = g == 0 ? l : 0.0f;
 }
 
-// The launch arguments of a kernel that appends, as they lie in its argument
-// block.  late_args() reads them where they are used: after the tile loop, or
-// in the one step that patches a page.  Taken from the kernel's parameters
-// they were held in scalar registers through the loop, which spilled 20-50 of
-// them (a 512-token chunk of 8192 keys: 101.0 -> 98.0 us).
-struct AppendKernelArgs {
-    AttnParams p;
+// The launch arguments as they lie in a kernel's argument block (pa where it
+// appends).  late_args() reads them where they are used: after the tile loop,
+// or in the one step that patches a page.  Taken from the kernel's parameters
+// they are held in scalar registers through the loop (head_dim 128: 97 instead
+// of 76, and 20-50 spilled in the forms that append: a 512-token chunk of 8192
+// keys 101.0 -> 98.0 us).
+struct KernelArgs {
     PrefillGrid gr;
+    AttnParams p;
     PrefillAppend pa;
 };
-__device__ __forceinline__ const AppendKernelArgs& late_args() {
-    typedef const __attribute__((address_space(4))) AppendKernelArgs args_t;
+__device__ __forceinline__ const KernelArgs& late_args() {
+    typedef const __attribute__((address_space(4))) KernelArgs args_t;
     args_t* a = (args_t*)__builtin_amdgcn_kernarg_segment_ptr();
     __asm__ volatile("" : "+s"(a));
-    return *(const AppendKernelArgs*)a;
+    return *(const KernelArgs*)a;
 }
 
 // The op's append, inside the attention launch: the chunk's K and V rows
@@ -234,7 +243,7 @@ __device__ __forceinline__ const AppendKernelArgs& late_args() {
 constexpr int kCopy = 4;
 template <int D>
 __device__ __forceinline__ void append_chunk(int tid, int n_threads) {
-    const AppendKernelArgs& a = late_args();
+    const KernelArgs& a = late_args();
     const AttnParams& p = a.p;
     const PrefillGrid& gr = a.gr;
     const PrefillAppend& pa = a.pa;
@@ -592,6 +601,8 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
         step(std::bool_constant<kNew>{}, t + 1, buf1, buf0);
     }
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // the trailing (empty) loads have landed: LDS is free
+    const AttnParams& pl = late_args().p;
+    const PrefillGrid& gl = late_args().gr;
 
     // Keys of a masked half that a query may not see meet a zero probability
     // in the P.V MFMA, and 0 x NaN is NaN: a NaN or infinite V row there would
@@ -610,7 +621,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
             for (int i = 0; i < 4; ++i) tsum += acc[db][i];
         if (__any(!(fabsf(tsum) <= __FLT_MAX__))) {
             float res[DB * 4 + 2];
-            prefill_exact_part<D, F16, KT, kNew>(p, qrow, head_off, hkv, s_row, kh, wave_end, t_begin, t_end, res);
+            prefill_exact_part<D, F16, KT, kNew>(pl, qrow, head_off, hkv, s_row, kh, wave_end, t_begin, t_end, res);
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -668,8 +679,8 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     if (r_out >= R) return;
     if constexpr (kSplit) {
         // partials: o [split][unit][row][D], then {m, l} [split][unit][row]
-        const int64_t at = (int64_t(sp) * units + unit) * R + r_out;
-        float* const po = gr.partial + at * D + 4 * g;
+        const int64_t at = (int64_t(sp) * gl.units + unit) * R + r_out;
+        float* const po = gl.partial + at * D + 4 * g;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
             f32x4_t o;
@@ -678,13 +689,13 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
             *reinterpret_cast<f32x4_t*>(po + 16 * db) = o;
         }
         if (g == 0)
-            *reinterpret_cast<float2*>(gr.partial + int64_t(gr.n_splits) * units * R * D + 2 * at) = make_float2(mt, lt);
+            *reinterpret_cast<float2*>(gl.partial + int64_t(gl.n_splits) * gl.units * R * D + 2 * at) = make_float2(mt, lt);
         return;
     }
     const float inv = 1.0f / lt;
-    const int s_out = gr.by_pack(r_out);
-    uint16_t* orow = p.out + bat * gr.o_batch + int64_t(hg * pack + (r_out - s_out * pack)) * p.o_head_stride +
-                     int64_t(s_out) * p.o_tok_stride;
+    const int s_out = gl.by_pack(r_out);
+    uint16_t* orow = pl.out + bat * gl.o_batch + int64_t(hg * gl.pack + (r_out - s_out * gl.pack)) * pl.o_head_stride +
+                     int64_t(s_out) * pl.o_tok_stride;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
         float o[4];
@@ -707,7 +718,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
 // form of one 128 KB, 196-VGPR workgroup per CU running two query tiles of
 // 2 x 32 queries, A/B on one box); D = 256: 128 KB, one workgroup per CU.
 template <bool F16, bool kSplit, bool kNew>
-__global__ __launch_bounds__(512, kNew ? 4 : 2) void paged_prefill_d128_kernel(AttnParams p, PrefillGrid gr, AppendArg<kNew>) {
+__global__ __launch_bounds__(512, kNew ? 4 : 2) void paged_prefill_d128_kernel(PrefillGrid gr, AttnParams p, AppendArg<kNew>) {
     prefill_tiles<128, F16, kSplit, 2, kNew>(p, gr);
 }
 // 16 waves on 128-key tiles, one workgroup per CU: the same waves per CU as
@@ -721,11 +732,11 @@ __global__ __launch_bounds__(512, kNew ? 4 : 2) void paged_prefill_d128_kernel(A
 // 16.0 against 15.6, 600 of 1500 18.9 against 19.7; 40 of 40: 8.7 against 6.3).
 constexpr int kWideFrom = 1280;
 template <bool F16, bool kNew>
-__global__ __launch_bounds__(1024) void paged_prefill_d128_wide_kernel(AttnParams p, PrefillGrid gr, AppendArg<kNew>) {
+__global__ __launch_bounds__(1024) void paged_prefill_d128_wide_kernel(PrefillGrid gr, AttnParams p, AppendArg<kNew>) {
     prefill_tiles<128, F16, false, 4, kNew>(p, gr);
 }
 template <bool F16, bool kSplit, bool kNew>
-__global__ __launch_bounds__(512) void paged_prefill_d256_kernel(AttnParams p, PrefillGrid gr, AppendArg<kNew>) {
+__global__ __launch_bounds__(512) void paged_prefill_d256_kernel(PrefillGrid gr, AttnParams p, AppendArg<kNew>) {
     prefill_tiles<256, F16, kSplit, 2, kNew>(p, gr);
 }
 
@@ -797,7 +808,7 @@ int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, const AppendArg
     const int64_t rows = int64_t(p.S) * gr.pack, units = gr.units;
     const int64_t wgs = gr.n_rt * units * gr.n_splits;
     const bool split = gr.n_splits > 1;
-    void (*k)(AttnParams, PrefillGrid, AppendArg<kNew>);
+    void (*k)(PrefillGrid, AttnParams, AppendArg<kNew>);
     int threads = 512;
     if constexpr (D == 128) {
         k = split ? paged_prefill_d128_kernel<F16, true, kNew> : paged_prefill_d128_kernel<F16, false, kNew>;
@@ -808,7 +819,7 @@ int launch_prefill_d(const AttnParams& p, const PrefillGrid& gr, const AppendArg
     } else {
         k = split ? paged_prefill_d256_kernel<F16, true, kNew> : paged_prefill_d256_kernel<F16, false, kNew>;
     }
-    hipLaunchKernelGGL(k, dim3(unsigned(wgs)), dim3(threads), 0, stream, p, gr, pa);
+    hipLaunchKernelGGL(k, dim3(unsigned(wgs)), dim3(threads), 0, stream, gr, p, pa);
     GENLLM_LAUNCH_CHECK("paged_prefill kernel");
     if (!split) return GENLLM_OK;
     constexpr int kMergeWgRows = kMergeThreads / (D / 4);
