@@ -641,18 +641,29 @@ __global__ __launch_bounds__(W * 64) void paged_decode_kernel(const int32_t* k_i
         float L = 0.0f, O0[VH], O1[VH];
 #pragma unroll
         for (int hh = 0; hh < VH; ++hh) O0[hh] = O1[hh] = 0.0f;
-        // A wave without a maximum has weight 0, multiplied all the same: its l
-        // and o are zeros if the row sees none of its keys, NaN if every score
-        // is NaN.
-        const float ref = M == -INFINITY ? 0.0f : M;
+        if (M != -INFINITY) {
 #pragma unroll
-        for (int w2 = w0; w2 < w0 + WP; ++w2) {
-            const float e = exp2_fast(lds_m[w2][ri] - ref);
-            L += lds_l[w2][ri] * e;
+            for (int w2 = w0; w2 < w0 + WP; ++w2) {
+                const float e = exp2_fast(lds_m[w2][ri] - M);
+                L += lds_l[w2][ri] * e;
 #pragma unroll
-            for (int hh = 0; hh < VH; ++hh) {
-                O0[hh] += lds_o[w2][ri][128 * hh + 2 * lane] * e;
-                O1[hh] += lds_o[w2][ri][128 * hh + 2 * lane + 1] * e;
+                for (int hh = 0; hh < VH; ++hh) {
+                    O0[hh] += lds_o[w2][ri][128 * hh + 2 * lane] * e;
+                    O1[hh] += lds_o[w2][ri][128 * hh + 2 * lane + 1] * e;
+                }
+            }
+        } else {
+            // no wave has a maximum: its l and o are zeros if the row sees none
+            // of the keys, NaN if every score is NaN.  (Apart: with one loop
+            // for both, 16 rows of 76 keys took 6.11 instead of 5.99 us.)
+#pragma clang loop unroll(disable)
+            for (int w2 = w0; w2 < w0 + WP; ++w2) {
+                L += lds_l[w2][ri];
+#pragma unroll
+                for (int hh = 0; hh < VH; ++hh) {
+                    O0[hh] += lds_o[w2][ri][128 * hh + 2 * lane];
+                    O1[hh] += lds_o[w2][ri][128 * hh + 2 * lane + 1];
+                }
             }
         }
         if (p.n_splits == 1) {
