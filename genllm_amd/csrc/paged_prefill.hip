@@ -21,10 +21,10 @@
 // against 31.5 us at config 4 and 47.4 against 48.1 us at head_dim 256 with
 // the halves of two row blocks paired instead); the two halves of a row
 // block are merged through LDS at the end.  At
-// head_dim 128 a workgroup holds 64 KB of LDS and at most 128 VGPRs per lane,
+// head_dim 128 a workgroup holds 66 KB of LDS and at most 128 VGPRs per lane,
 // so two workgroups share a CU (4 waves per SIMD: one workgroup's barrier
 // waits and dependent chains are filled by the other's work); the grid's
-// order puts a long and a short row tile on each CU.  At head_dim 256 (128
+// order puts a long and a short row tile on each CU.  At head_dim 256 (130
 // KB) one workgroup runs per CU.
 // Key tiles are staged in two LDS buffers (one tile in flight while the other
 // is computed), K and V each as [token][dim] rows whose 16-byte chunks are
@@ -47,7 +47,7 @@
 //        P^T is the lane's own 8 exponentials; A = V^T from two
 //        ds_read_b64_tr_b16 per 16 dims).  O^T[dim][q] belongs to the lane's
 //        own query column, so the rescale by 2^(m_old-m_new) stays lane-local.
-// Causal masking is applied only to the key halves that reach past the first
+// Causal masking is applied only to the key parts that reach past the first
 // query of the wave (the diagonal) or past the cache end.
 #include <climits>
 #include <type_traits>
@@ -362,9 +362,9 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
                          : p.causal     ? min(qabs0 + gr.by_pack(min(q0 + QW, R) - 1) + 1, kv_end)
                                         : kv_end;
 
-    // ---- staging: wave w < 4 moves page w of each tile, its K rows, then its
-    // V rows; waves 4-7 issue no tile loads.  Waves 4-7 share their SIMDs
-    // with waves 0-3 and reach their S^T MFMAs after them, so the step waits
+    // ---- staging: wave w < KP moves page w of each tile, its K rows, then its
+    // V rows; the other half of the waves issue no tile loads.  (8 waves:) waves
+    // 4-7 share their SIMDs with waves 0-3 and reach their S^T MFMAs after them, so the step waits
     // for them: keeping the loads' issue off their path measured 31.3 against
     // 31.5 us at config 4 and 48.9 against 50.2 us at head_dim 256 (A/B on one
     // box; the mirror split, waves 4-7 loading, 32.2 and 50.7).  Every K row
@@ -470,7 +470,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     const float c = fmaxf(p.scale_log2, __FLT_MIN__);  // > 0: masked -inf scores give exactly 0
     const float inv_c = 1.0f / c;                       // may be inf (then no row grows after its first tile)
     auto compute_tile = [&](int t, const lds_char* buf, bool masked, auto&& after_s) {
-        const int tok0 = t * KT + KH * kh;  // first key of the half
+        const int tok0 = t * KT + KH * kh;  // first key of the part
         const int r0 = KH * kh;             // its first LDS row (a multiple of 16)
         f32x4_t s[2] = {f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}};
 #pragma unroll
@@ -498,7 +498,7 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
                                                  __builtin_elementwise_maximum(s[0][2], s[0][3]));
         mx = __builtin_elementwise_maximum(mx, __builtin_elementwise_maximum(__builtin_elementwise_maximum(s[1][0], s[1][1]),
                                                                              __builtin_elementwise_maximum(s[1][2], s[1][3])));
-        if (__any(mx > th)) {  // lazy rescale, as in the D = 128 kernel
+        if (__any(mx > th)) {  // lazy rescale, as in the decode kernel
             mx = fmaxf(mx, __shfl_xor(mx, 16));
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             const bool grow = mx > th;
@@ -541,9 +541,9 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     // ---- pipeline: one barrier per tile, two buffers.  Step t waits for its
     // own loads of tile t, meets the other waves (tile t complete in LDS;
     // everybody done with tile t-1), starts tile t+1 into the other buffer,
-    // then computes its half of tile t.  Every step issues the same 8 loads
-    // in each loading wave; a tile past the last one has no rows below kv_end and reads
-    // as zeros.  Page ids arrive IDS_BLOCK tiles per load; the rare reload
+    // then computes its key part of tile t.  Every step issues the same 2 NI
+    // loads in each loading wave; a tile past the last one has no rows below
+    // kv_end and reads as zeros.  Page ids arrive IDS_BLOCK tiles per load; the rare reload
     // drains the loads in flight.
     const int t_ids = t_begin & ~(IDS_BLOCK - 1);
     int ids0 = paged && dma_wave ? load_ids(t_ids, 0) : 0;
@@ -607,9 +607,10 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     // Keys of a masked half that a query may not see meet a zero probability
     // in the P.V MFMA, and 0 x NaN is NaN: a NaN or infinite V row there would
     // reach queries the reference never lets it reach.  A wave whose state
-    // came out NaN or infinite (only ever with such inputs) forms its key half
-    // again from the pools, in fp32, visiting for each query only the keys it
-    // sees, as the reference's loop does.  The check is one sum of the state
+    // came out NaN or infinite (only ever with such inputs) forms its key part
+    // again from the pools (the chunk's keys, in the forms that append, from
+    // k_new / v_new), in fp32, visiting for each query only the keys it sees, as
+    // the reference's loop does.  The check is one sum of the state
     // (a NaN or an infinity in it makes the sum non-finite); measured at
     // config 4, 30.85-30.93 against 30.65-30.80 us (A/B on one box, two passes;
     // checking each value instead cost 0.3-0.4 us).
@@ -713,10 +714,10 @@ __device__ __forceinline__ void prefill_tiles(const AttnParams& p, const Prefill
     }
 }
 
-// D = 128: 64 KB of LDS and at most 128 VGPRs, so two workgroups share a CU
+// D = 128: 66 KB of LDS and at most 128 VGPRs, so two workgroups share a CU
 // (4 waves per SIMD: at config 4 36.2 us, against 41.9 us for the earlier
 // form of one 128 KB, 196-VGPR workgroup per CU running two query tiles of
-// 2 x 32 queries, A/B on one box); D = 256: 128 KB, one workgroup per CU.
+// 2 x 32 queries, A/B on one box); D = 256: 130 KB, one workgroup per CU.
 template <bool F16, bool kSplit, bool kNew>
 __global__ __launch_bounds__(512, kNew ? 4 : 2) void paged_prefill_d128_kernel(PrefillGrid gr, AttnParams p, AppendArg<kNew>) {
     prefill_tiles<128, F16, kSplit, 2, kNew>(p, gr);
